@@ -233,16 +233,17 @@ constexpr int kCombineThreads = 256;
 constexpr int kMaxSplits = 512;
 
 // ---------------------------------------------------------------------------
-// Balanced decode splits.  A decode launch has U = S * B workgroups per group
-// of kv heads; with every sequence split S ways, a batch of one long context
-// and many short ones leaves most of them idle while the long one streams.
-// Instead the U units go to the batch's pages: P, the pages per unit, is the
-// smallest value (at least ceil(max pages / kMaxSplits), so that no row has
-// more partials than the combine takes) with sum_b ceil(pages_b / P) <= U,
-// and sequence b gets ceil(pages_b / P) consecutive units.  A uniform batch
-// gets S units per sequence, the page ranges of the plain split.  Unit u's
-// partial of head h sits at slot h * U + u, so a row's partials are
-// consecutive, as in the plain layout.  Each function is evaluated by a
+// Balanced decode splits.  With every sequence split S ways, a batch of one
+// long context and many short ones leaves most workgroups idle while the long
+// one streams.  Instead the launch has U = p.units workgroups per group of kv
+// heads (decode_units: one grid round, not a multiple of B) and they go to the
+// batch's pages: P, the pages per unit, is the smallest value (at least
+// ceil(max pages / kMaxSplits), so that no row has more partials than the
+// combine takes) with sum_b ceil(pages_b / P) <= U, and sequence b gets
+// ceil(pages_b / P) consecutive units.  A uniform batch gets floor(U / B)
+// units per sequence, the page ranges of the plain split.  Unit u's partial of
+// head h sits at slot h * U + u, so a row's partials are consecutive, as in
+// the plain layout.  Each function is evaluated by a
 // whole wave (lane b holds sequence b: batches of up to kBalSeqs) and returns
 // the same value in every lane.
 //
@@ -278,17 +279,19 @@ __device__ __forceinline__ BatchPages batch_pages(const Params& p) {
   bp.pg = decode_pages(p, bp.ctx);
   return bp;
 }
-// P for S units per sequence of a B-sequence batch (U = S * B).
-__device__ int decode_unit_pages(const BatchPages& bp, int S, int B) {
+// P for U units over a B-sequence batch (U >= B).
+__device__ int decode_unit_pages(const BatchPages& bp, int U, int B) {
   const int lane = threadIdx.x & 63;
   const int mx = __ockl_wfred_max_i32(bp.pg);
   const int mn = __ockl_wfred_min_i32(lane < B ? bp.pg : INT_MAX);
   int lo = max(1, (mx + kMaxSplits - 1) / kMaxSplits);
-  // Every sequence the same length: S units each, the plain split.
-  if (mn == mx) return max(lo, (mx + S - 1) / S);
+  // Every sequence the same length: floor(U / B) units each, the plain split.
+  if (mn == mx) {
+    const int S = U / B;
+    return max(lo, (mx + S - 1) / S);
+  }
   const int tot = __ockl_wfred_add_i32(bp.pg);
   const int nz = __ockl_wfred_add_i32(bp.pg > 0 ? 1 : 0);
-  const int U = S * B;
   // Bounds on the answer: a P that fits has tot / P <= U, so P >= ceil(tot / U);
   // P = mx fits (at most B <= U units), and so does ceil(tot / (U - nz)) when
   // U > nz, since sum ceil(pages / P) <= tot / P + nz.
@@ -395,14 +398,14 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(Params p) {
   }
   const int tid = threadIdx.x, lane = tid & 63;
   // The row's partials: S of them at row * S + s, or, with balanced decode
-  // splits, n_s at h * S * B + u0 + s (its sequence's units).
+  // splits, n_s at h * units + u0 + s (its sequence's units).
   __shared__ int s_first, s_count;
   int64_t first = row * S;
   int n_s = S;
   if (p.balanced) {
     if (tid < 64) {
       const BatchPages bp = batch_pages(p);
-      const int P = decode_unit_pages(bp, S, p.B);
+      const int P = decode_unit_pages(bp, p.units, p.B);
       int u0, n;
       decode_units_of_seq(bp, P, b, &u0, &n);
       if (tid == 0) {
@@ -411,7 +414,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(Params p) {
       }
     }
     __syncthreads();
-    first = (int64_t)h * S * p.B + s_first;
+    first = (int64_t)h * p.units + s_first;
     n_s = s_count;
   }
   i += p.q0_off;  // rows of a dense split start at position q0_off
@@ -799,12 +802,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   T* vtile = vtile_all[wave];
   T* qtile = qtile_all[wave];
   const int S = p.num_splits;
-  const int unit = blockIdx.y * S + blockIdx.x;  // balanced splits: this workgroup's unit
+  const int unit = blockIdx.x;  // balanced splits: this workgroup's unit
   int b = blockIdx.y, split = blockIdx.x, per = 0;
   int ctx;
   if (p.balanced) {
     const BatchPages bp = batch_pages(p);
-    per = decode_unit_pages(bp, S, p.B);
+    per = decode_unit_pages(bp, p.units, p.B);
     if (!decode_seq_of_unit(bp, per, unit, &b, &split)) return;  // past the batch's units: no partial to write
     // Wave-uniform results, kept in scalar registers so that the page loop's
     // bounds and page-table reads stay scalar (as vector loads they would
@@ -997,7 +1000,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       *reinterpret_cast<vec4*>(dst + 16 * blk) = ov;
     }
   } else {
-    const int64_t slot = p.balanced ? (int64_t)head * S * p.B + unit : row_id(p, b, 0, head) * S + split;
+    const int64_t slot = p.balanced ? (int64_t)head * p.units + unit : row_id(p, b, 0, head) * S + split;
     float* dst = p.ws_o + slot * 128 + 4 * grp;
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk];
@@ -1036,12 +1039,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   if (g >= p.Hkv) return;  // no workgroup barriers below
   float* vtile = vtile_all[wave];
   const int S = p.num_splits;
-  const int unit = blockIdx.y * S + blockIdx.x;  // balanced splits: this workgroup's unit
+  const int unit = blockIdx.x;  // balanced splits: this workgroup's unit
   int b = blockIdx.y, split = blockIdx.x, per = 0;
   int ctx;
-  if (p.balanced) {
+  const bool balanced = PREF > 1 && p.balanced;  // the one-block instance is launched unbalanced only
+  if (balanced) {
     const BatchPages bp = batch_pages(p);
-    per = decode_unit_pages(bp, S, p.B);
+    per = decode_unit_pages(bp, p.units, p.B);
     if (!decode_seq_of_unit(bp, per, unit, &b, &split)) return;  // past the batch's units: no partial to write
     // Wave-uniform results, kept in scalar registers so that the page loop's
     // bounds and page-table reads stay scalar (as vector loads they would
@@ -1059,7 +1063,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int lo = p.window > 0 ? max(0, ctx - p.window) : 0;
   const int pg_lo = lo >> 4;
   const int pg_hi = (ctx + 15) >> 4;
-  if (!p.balanced) per = (pg_hi - pg_lo + S - 1) / S;
+  if (!balanced) per = (pg_hi - pg_lo + S - 1) / S;
   const int p0 = pg_lo + split * per;
   const int p1 = min(pg_hi, p0 + per);
 
@@ -1211,7 +1215,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk] * il;
   } else {
-    const int64_t slot = p.balanced ? (int64_t)head * S * p.B + unit : row_id(p, b, 0, head) * S + split;
+    const int64_t slot = balanced ? (int64_t)head * p.units + unit : row_id(p, b, 0, head) * S + split;
     float* dst = p.ws_o + slot * 128 + 4 * grp;
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk];
@@ -1239,13 +1243,13 @@ int device_cus() {
   return v;
 }
 
-// Number of key splits per (sequence, kv-head group); identical for the
-// workspace query and the launch.  The default targets kDecWgsPerCu
-// workgroups per CU, so the decode grid runs as a single round (at batch 16
-// with 8 kv heads on 256 CUs: 16 splits of 512 pages; 32 splits, two rounds,
-// measured 3 % slower).
-int decode_splits(int B, int Hkv, int max_ctx, int page_size) {
-  const int target = env_int("KESSIE_DECODE_WGS", kDecWgsPerCu * device_cus());
+// Upper bound on a decode's key splits per (sequence, kv-head group), and the
+// splits of the partials-only form: what the workspace is sized and refused
+// by, and what kessie_fog_decode_num_splits reports.  decode_launch_splits
+// never exceeds it.
+int decode_target() { return env_int("KESSIE_DECODE_WGS", kDecWgsPerCu * device_cus()); }
+
+int decode_splits(int B, int Hkv, int max_ctx, int page_size, int target = decode_target()) {
   const int units = B * div_up(Hkv, kDecWaves);
   // Counted in 16-token blocks, the unit the MFMA decode streams (pages of
   // 16 * 2^k tokens hold 2^k of them); smaller pages count as they are.
@@ -1258,6 +1262,42 @@ int decode_splits(int B, int Hkv, int max_ctx, int page_size) {
   s = min(s, max(1, pages / 2));
   s = min(s, kMaxSplits);
   return max(s, 1);
+}
+
+// Key splits of a decode that merges its own partials.  The grid runs as one
+// round of kDecWgsPerCu workgroups per CU, so the share is rounded down: one
+// workgroup past the round waits for a whole split and runs almost alone.
+// bf16 steps with 8 kv heads, rounded up (1,056-1,152 workgroups on 1,024
+// slots) -> one round: 24 sequences of 500-16,384 tokens 115.4 -> 83.3 us, 3
+// of 60,000 176.4 -> 120.9, 9 of 12,800-128,000 444 -> 297; fp16 GQA 8, 12
+// sequences on a 4,096-token window 62.6 -> 46.8.  A window bounds the blocks
+// there are to split: decode_splits leaves a short window's splits mostly
+// empty (4 sequences, 1 kv head, window 1,024: 15.5 -> 14.4 us).
+// target: decode_target(); bound: decode_splits.
+int decode_launch_splits(int B, int Hkv, int max_ctx, int window, int page_size, int target, int bound) {
+  const int units = max(B * div_up(Hkv, kDecWaves), 1);
+  int s = target / units;
+  // Past half a round of units there is no second split to round down to: two
+  // splits, whose surplus fills in behind sequences that end early.
+  if (s < 2) s = div_up(target, units);
+  if (window > 0 && window < max_ctx) {
+    const int blk = max(min(page_size, 16), 1);
+    s = min(s, (div_up(window, blk) + 1) / 2);
+  }
+  return max(1, min(s, bound));
+}
+
+// Workgroups per group of kv heads of a balanced decode: the round of
+// decode_launch_splits, whole (not S times the batch), and never more than
+// the partials' bound of B * decode_splits.
+int decode_units(int B, int Hkv, int target, int bound) {
+  return max(B, min(target / max(div_up(Hkv, kDecWaves), 1), B * bound));
+}
+
+// Grid of a decode launch: splits x sequences, or the units of a balanced one.
+dim3 decode_grid(const Params& p) {
+  const int z = div_up(p.Hkv, kDecWaves);
+  return p.balanced ? dim3(p.units, 1, z) : dim3(p.num_splits, p.B, z);
 }
 
 // Key splits of the MFMA prefill: enough workgroups for one per CU (one fits a
@@ -1320,7 +1360,7 @@ int launch_decode_mfma(Params& p, hipStream_t stream) {
   // SIMD (measured at batch 16, 128K context: 1.308 ms against 1.314 ms with
   // four pages in flight -- which also cost one sequence 3-9 % -- and 1.398 ms
   // with two pages at three waves per SIMD).
-  dim3 grid(p.num_splits, p.B, div_up(p.Hkv, kDecWaves));
+  const dim3 grid = decode_grid(p);
   const int fog = (p.bias ? kFogBias : 0) | (p.vscale ? kFogVs : 0);
   const dim3 block(kDecWaves * 64);
   switch (fog) {
@@ -1368,12 +1408,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   if (g >= p.Hkv) return;  // no workgroup barriers below
   float* pslot = pslot_all[wave];
   const int S = p.num_splits;
-  const int unit = blockIdx.y * S + blockIdx.x;  // balanced splits: this workgroup's unit
+  const int unit = blockIdx.x;  // balanced splits: this workgroup's unit
   int b = blockIdx.y, split = blockIdx.x, per = 0;
   int ctx;
-  if (p.balanced) {
+  const bool balanced = PREF > 1 && p.balanced;  // the one-block instance is launched unbalanced only
+  if (balanced) {
     const BatchPages bp = batch_pages(p);
-    per = decode_unit_pages(bp, S, p.B);
+    per = decode_unit_pages(bp, p.units, p.B);
     if (!decode_seq_of_unit(bp, per, unit, &b, &split)) return;  // past the batch's units: no partial to write
     per = __builtin_amdgcn_readfirstlane(per);
     b = __builtin_amdgcn_readfirstlane(b);
@@ -1390,7 +1431,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int lo = p.window > 0 ? max(0, ctx - p.window) : 0;
   const int pg_lo = lo >> 4;
   const int pg_hi = (ctx + 15) >> 4;
-  if (!p.balanced) per = (pg_hi - pg_lo + S - 1) / S;
+  if (!balanced) per = (pg_hi - pg_lo + S - 1) / S;
   const int p0 = pg_lo + split * per;
   const int p1 = min(pg_hi, p0 + per);
 
@@ -1550,7 +1591,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       dst[lane] = oacc[0][r] * il;
       dst[64 + lane] = oacc[1][r] * il;
     } else {
-      const int64_t slot = p.balanced ? (int64_t)head * S * p.B + unit : row_id(p, b, 0, head) * S + split;
+      const int64_t slot = balanced ? (int64_t)head * p.units + unit : row_id(p, b, 0, head) * S + split;
       float* dst = p.ws_o + slot * 128;
       dst[lane] = oacc[0][r];
       dst[64 + lane] = oacc[1][r];
@@ -1572,7 +1613,7 @@ void launch_f32_instance(const Params& p, dim3 grid, dim3 block, hipStream_t str
 
 template <int G>
 int launch_decode_mfma_f32(Params& p, hipStream_t stream) {
-  dim3 grid(p.num_splits, p.B, div_up(p.Hkv, kDecWaves));
+  const dim3 grid = decode_grid(p);
   const int fog = (p.bias ? kFogBias : 0) | (p.vscale ? kFogVs : 0);
   const dim3 block(kDecWaves * 64);
   // Splits of at most two 16-token blocks (short contexts) take the
@@ -1739,7 +1780,9 @@ static int decode_entry(const void* q, const void* kv_pool, int num_pages, int64
                  "fog decode: page_table and ctx_lens are required");
   KESSIE_REQUIRE(kv_stride >= 0, KESSIE_ERR_INVALID, "fog decode: kv_stride %lld", (long long)kv_stride);
   if (batch == 0) return KESSIE_OK;
-  p.num_splits = decode_splits(batch, num_kv_heads, max_ctx, page_size);
+  const int target = decode_target();
+  const int bound = decode_splits(batch, num_kv_heads, max_ctx, page_size, target);
+  p.num_splits = bound;
   p.direct_out = (!partials_only && p.num_splits == 1) ? 1 : 0;
   p.launch_combine = partials_only ? 0 : 1;
   if (!p.direct_out) {
@@ -1747,19 +1790,26 @@ static int decode_entry(const void* q, const void* kv_pool, int num_pages, int64
     KESSIE_REQUIRE(workspace != nullptr && workspace_bytes >= need, KESSIE_ERR_WORKSPACE,
                    "fog decode: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     KESSIE_REQUIRE(aligned16(workspace), KESSIE_ERR_INVALID, "fog decode: workspace not 16-byte aligned");
-    carve_workspace(p, workspace, (int64_t)batch * num_q_heads);
+    carve_workspace(p, workspace, (int64_t)batch * num_q_heads);  // room for the bound's partials
   }
   hipStream_t s = as_stream(stream);
   if (decode_mfma_ok(p, dtype)) {
+    // The partials-only form and the generic kernel keep the bound's splits.
+    if (!partials_only && !p.direct_out) {
+      p.num_splits = decode_launch_splits(batch, num_kv_heads, max_ctx, window, page_size, target, bound);
+      p.direct_out = p.num_splits == 1 ? 1 : 0;
+    }
     // Split partials merged here: assign the splits by pages across the batch
     // (the partials-only form keeps the plain row * S + split layout).  Its
     // set-up costs each wave ~1 us before the first page load, so it is taken
-    // for batches of 2..kBalSeqs sequences whose bound on the K/V bytes (B *
-    // max_ctx tokens) streams for at least ~40 us, 256 MiB; one sequence, or a
-    // batch that small, gets the plain split.
-    const double kv_bound = (double)batch * max_ctx * num_kv_heads * head_dim * 2.0 * dtype_size(dtype);
+    // for batches of 2..kBalSeqs sequences whose bound on the K/V bytes (B
+    // times max_ctx tokens, or the window's) streams for at least ~40 us, 256
+    // MiB; one sequence, or a batch that small, gets the plain split.
+    const int seen = window > 0 ? min(window, max_ctx) : max_ctx;
+    const double kv_bound = (double)batch * seen * num_kv_heads * head_dim * 2.0 * dtype_size(dtype);
     p.balanced = (!partials_only && !p.direct_out && batch >= 2 && batch <= kBalSeqs &&
                   kv_bound >= 256.0 * 1024 * 1024) ? 1 : 0;
+    p.units = p.balanced ? decode_units(batch, num_kv_heads, target, bound) : 0;
     if (dtype == KESSIE_DTYPE_F32) return run_decode_mfma_f32(p, s);
     return dtype == KESSIE_DTYPE_BF16 ? run_decode_mfma<bf16_t>(p, s) : run_decode_mfma<f16_t>(p, s);
   }

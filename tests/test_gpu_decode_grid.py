@@ -1,0 +1,39 @@
+"""GPU parity of the decode's one-round grid: splits rounded down to the chip's
+workgroup slots, balanced units that are no multiple of the batch, and splits
+bounded by a window.  |gpu - ref| <= 2e-2 + 1e-2 * |ref| (bf16 probabilities
+and outputs, fp32 sums), as tests/test_gpu_decode.py."""
+import pytest
+import torch
+
+from oracle.attention import paged_decode_ref
+from tests.inputs import decode_case, gen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,hkv,ctx,lens,window", [
+    (3, 8, 32768, [32768, 1, 9000], 0),                     # balanced: 256 units over 3 sequences
+    (7, 2, 40000, [40000, 0, 17, 16, 15, 2500, 700], 0),    # balanced, one group of kv heads, an empty sequence
+    (64, 8, 2048, [2048] * 5 + list(range(1, 60)), 0),      # balanced at the largest batch it takes
+    (5, 8, 3000, [3000, 1500, 31, 2999, 16], 1024),         # a window bounds the splits
+    (4, 1, 9000, [9000, 8999, 33, 1], 33),                  # ... to two of them
+    (3, 1, 4000, [4000, 40, 17], 5),                        # ... and to one (no partials)
+    (130, 8, 64, [64] * 100 + [1 + i for i in range(30)], 0),  # past half a round: two splits
+])
+def test_decode_one_round_grid(dev, b, hkv, ctx, lens, window):
+    from kessie_amd import ops
+
+    q, pool, table, lens_d = decode_case(b, 4 * hkv, hkv, 128, ctx, 16, torch.bfloat16, dev, seed=41, ctx_lens=lens)
+    vs = torch.rand(ctx, generator=gen(dev, 42), device=dev)
+    out = ops.fog_decode(q, pool, table, lens_d, ctx, fog_vscale=vs, window=window)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out.float()).all()
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        row = table[i].long()[: -(-n // 16)]
+        ref = paged_decode_ref(q[i:i + 1].cpu(), pool[row].cpu(), torch.arange(len(row), dtype=torch.int32)[None],
+                               torch.tensor([n]), vs.cpu(), None, window)
+        diff = (out[i:i + 1].float().cpu() - ref).abs()
+        assert bool((diff <= 2e-2 + 1e-2 * ref.abs()).all()), f"sequence {i} ({n} tokens): {diff.max().item():.3e}"
