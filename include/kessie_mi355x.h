@@ -219,8 +219,8 @@ size_t kessie_fog_prefill_workspace_bytes(int batch, int num_q_tokens,
  * j <= q_pos (causal) with (window == 0 or q_pos - j < window), fog as in
  * decode, fog index = key position.  q/out: [B][C][Hq][D] contiguous.  This
  * equals the last C rows of the reference's dense math over ctx tokens
- * (kessie_hip_kernels.py:577-593).  Kernels: bf16/fp16 on MFMA (head_dim 128,
- * pages of 16 * 2^k tokens, GQA 1/2/4/8/16), fp32 on fp32 MFMA (head_dim 128,
+ * (kessie_hip_kernels.py:577-593).  Kernels: bf16/fp16 on MFMA (head_dim 128
+ * or 64, pages of 16 * 2^k tokens, GQA up to 16), fp32 on fp32 MFMA (head_dim 128,
  * same pages, GQA up to 128), everything else on the generic kernel. */
 int kessie_fog_prefill_paged(
     const void* q, const void* kv_pool, int num_pages, int64_t page_stride,
@@ -251,6 +251,20 @@ int kessie_fog_prefill_paged(
  * max_query_len, ...) and used only when the chunks are too few to fill the
  * device (split-K). */
 int kessie_fog_prefill_varlen(
+    const void* q, const int32_t* query_start_loc, int max_query_len,
+    const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
+    int64_t kv_stride, int64_t head_stride, const int32_t* page_table,
+    int64_t table_stride, const int32_t* ctx_lens, const float* fog_vscale,
+    int64_t fog_vscale_bstride, const float* fog_bias, int64_t fog_bias_bstride,
+    void* out, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+    int page_size, int max_ctx, int window, float sm_scale, int causal,
+    int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/* kessie_fog_prefill_varlen for every shape of the MFMA kernels: also head_dim
+ * 64 and GQA ratios up to 16 that are no power of two (bf16/fp16), which the
+ * other entry reports as unsupported.  Same arguments, semantics and
+ * workspace. */
+int kessie_fog_prefill_batch(
     const void* q, const int32_t* query_start_loc, int max_query_len,
     const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
     int64_t kv_stride, int64_t head_stride, const int32_t* page_table,

@@ -2094,14 +2094,16 @@ extern "C" int kessie_fog_prefill_paged(const void* q, const void* kv_pool, int 
   return run_generic(dtype, p, as_stream(stream));
 }
 
-extern "C" int kessie_fog_prefill_varlen(const void* q, const int32_t* query_start_loc, int max_query_len,
-                                         const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
-                                         int64_t kv_stride, int64_t head_stride, const int32_t* page_table,
-                                         int64_t table_stride, const int32_t* ctx_lens, const float* fog_vscale,
-                                         int64_t fog_vscale_bstride, const float* fog_bias, int64_t fog_bias_bstride,
-                                         void* out, int batch, int num_q_heads, int num_kv_heads, int head_dim,
-                                         int page_size, int max_ctx, int window, float sm_scale, int causal,
-                                         int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+// Variable-length prefill.  any_shape false: the shapes kessie_fog_prefill_varlen has always taken (callers run
+// the others per sequence when it reports them unsupported); true: every shape of the MFMA kernels.
+static int prefill_varlen_entry(const void* q, const int32_t* query_start_loc, int max_query_len, const void* kv_pool,
+                                int num_pages, int64_t page_stride, int64_t tok_stride, int64_t kv_stride,
+                                int64_t head_stride, const int32_t* page_table, int64_t table_stride,
+                                const int32_t* ctx_lens, const float* fog_vscale, int64_t fog_vscale_bstride,
+                                const float* fog_bias, int64_t fog_bias_bstride, void* out, int batch,
+                                int num_q_heads, int num_kv_heads, int head_dim, int page_size, int max_ctx,
+                                int window, float sm_scale, int causal, int dtype, void* workspace,
+                                size_t workspace_bytes, void* stream, bool any_shape) {
   using namespace kessie;
   using namespace kessie::attn;
   clear_error();
@@ -2147,11 +2149,42 @@ extern "C" int kessie_fog_prefill_varlen(const void* q, const int32_t* query_sta
   KESSIE_REQUIRE(kv_stride >= 0, KESSIE_ERR_INVALID, "fog prefill varlen: kv_stride %lld", (long long)kv_stride);
   if (batch == 0 || max_query_len == 0) return KESSIE_OK;
   if (prefill_f32_ok(p, dtype)) return run_prefill_f32(p, workspace, workspace_bytes, stream);
-  KESSIE_REQUIRE(prefill_mfma_ok(p, dtype), KESSIE_ERR_UNSUPPORTED,
+  const bool listed = p.D == 128 && (p.G & (p.G - 1)) == 0;
+  KESSIE_REQUIRE((any_shape || listed) && prefill_mfma_ok(p, dtype), KESSIE_ERR_UNSUPPORTED,
                  "fog prefill varlen: shape not taken by the MFMA kernels (bf16/fp16: head_dim 128, pages of 16*2^k "
                  "tokens, GQA 1/2/4/8/16; fp32: head_dim 128, pages of 16*2^k tokens, GQA up to 128; 16-byte aligned "
                  "rows)");
   return run_prefill_mfma(p, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int kessie_fog_prefill_varlen(const void* q, const int32_t* query_start_loc, int max_query_len,
+                                         const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
+                                         int64_t kv_stride, int64_t head_stride, const int32_t* page_table,
+                                         int64_t table_stride, const int32_t* ctx_lens, const float* fog_vscale,
+                                         int64_t fog_vscale_bstride, const float* fog_bias, int64_t fog_bias_bstride,
+                                         void* out, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                         int page_size, int max_ctx, int window, float sm_scale, int causal,
+                                         int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  return prefill_varlen_entry(q, query_start_loc, max_query_len, kv_pool, num_pages, page_stride, tok_stride,
+                              kv_stride, head_stride, page_table, table_stride, ctx_lens, fog_vscale,
+                              fog_vscale_bstride, fog_bias, fog_bias_bstride, out, batch, num_q_heads, num_kv_heads,
+                              head_dim, page_size, max_ctx, window, sm_scale, causal, dtype, workspace,
+                              workspace_bytes, stream, false);
+}
+
+extern "C" int kessie_fog_prefill_batch(const void* q, const int32_t* query_start_loc, int max_query_len,
+                                        const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
+                                        int64_t kv_stride, int64_t head_stride, const int32_t* page_table,
+                                        int64_t table_stride, const int32_t* ctx_lens, const float* fog_vscale,
+                                        int64_t fog_vscale_bstride, const float* fog_bias, int64_t fog_bias_bstride,
+                                        void* out, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                        int page_size, int max_ctx, int window, float sm_scale, int causal, int dtype,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  return prefill_varlen_entry(q, query_start_loc, max_query_len, kv_pool, num_pages, page_stride, tok_stride,
+                              kv_stride, head_stride, page_table, table_stride, ctx_lens, fog_vscale,
+                              fog_vscale_bstride, fog_bias, fog_bias_bstride, out, batch, num_q_heads, num_kv_heads,
+                              head_dim, page_size, max_ctx, window, sm_scale, causal, dtype, workspace,
+                              workspace_bytes, stream, true);
 }
 
 // Reference launchers (kessie_kernels_v2.hip:716-751, 788-825): dense fp16

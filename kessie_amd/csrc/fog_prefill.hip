@@ -1,5 +1,9 @@
-// Chunked-prefill fog attention on MFMA for gfx950 (bf16 / f16, head_dim 128,
-// pages of 16 * 2^k tokens, GQA ratio 1/2/4/8/16, sm_scale > 0).
+// Chunked-prefill fog attention on MFMA for gfx950 (bf16 / f16, head_dim 128 or
+// 64, pages of 16 * 2^k tokens, GQA ratios up to 16, sm_scale > 0).  The GQA
+// ratio is a kernel argument: it is read before the loop only, and one
+// instance for all of them runs as fast as one per ratio (2,048 queries on
+// 131,072 tokens at GQA 4: 4.13 ms both).  Ratios that do
+// not divide 256 leave the rows past 256 / G * G of a workgroup idle.
 //
 // Math: the last C rows of kessie_hip_kernels.py:577-593 over ctx = L + C
 // tokens (query i at position ctx-C+i, causal, window, fog weights scaling V
@@ -31,6 +35,14 @@
 // sits on one XCD and the query tiles of that head share its keys in L2.
 //
 // Variants (template and Params):
+//   kExactP  the probabilities enter PV as two operands of T, the rounded value
+//            and what the rounding left (p to 2^-16 relative in bf16, 2^-22 in
+//            fp16), the V-fog weights multiply them in fp32 and V is not
+//            rescaled.  Twice the PV MFMAs, for the precision of the fp32 VALU
+//            kernel (attn_generic_kernel), which these shapes would otherwise
+//            take: 2,048 queries on 32,768 tokens at head_dim 64 49.3 ms there,
+//            0.96 ms (557 TFLOP/s) here; on 16,384 at 24 q / 8 kv heads of 128
+//            44.2 against 0.89 ms;
 //   kSplit   grid z splits each query tile's key tiles (split s takes tiles
 //            s, s + S, ...); every split stores unnormalised partials (O,
 //            max, sum) merged by the combine kernel -- used when the chunks
@@ -56,13 +68,16 @@ constexpr int kPfRows = kPfWaves * 32;  // query rows (position, head) per workg
 constexpr int kPfKT = 64;               // keys per tile (4 pages)
 constexpr int kPfStages = 4;            // LDS ring depth (a power of two)
 constexpr int kVRowW = kPfKT / 2 + 8;   // V^T tile row stride (32-bit words)
-// LDS geometry for head_dim D: 128, or 64 (the dense launchers only).
+// LDS geometry for head_dim D (128 or 64).
 template <int D>
 struct PfGeom {
   static constexpr int kKRow = D + 8;            // K tile row stride (elements)
   static constexpr int kKStage = kPfKT * kKRow;  // elements per K stage
   static constexpr int kVStage = D * kVRowW;     // words per V^T stage
-  static constexpr size_t kLdsBytes = (size_t)kPfStages * (kKStage * 2 + kVStage * 4 + kPfKT * 4);
+  // K, V^T, bias; the exact-P instances also keep the tile's V weights.
+  static constexpr size_t lds_bytes(bool exact_p) {
+    return (size_t)kPfStages * (kKStage * 2 + kVStage * 4 + kPfKT * 4 * (exact_p ? 2 : 1));
+  }
 };
 constexpr float kLog2e = 1.4426950408889634f;
 // Word 3 of a raw (unformatted, stride 0) buffer resource on gfx9-family parts.
@@ -117,6 +132,16 @@ __device__ __forceinline__ uint32_t pack2<f16_t>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
 }
 
+// The two halves of a packed dword, widened.
+template <typename T>
+__device__ __forceinline__ float unpack_lo(uint32_t w) {
+  return to_f32(__builtin_bit_cast(T, (uint16_t)w));
+}
+template <typename T>
+__device__ __forceinline__ float unpack_hi(uint32_t w) {
+  return to_f32(__builtin_bit_cast(T, (uint16_t)(w >> 16)));
+}
+
 // max(a, b, c) in one instruction.  fmaxf on MFMA results first quiets each
 // input (one extra v_max per score); scores hold no signalling NaN, so the
 // raw instruction gives the same result.  Being inline assembly, it gets no
@@ -159,9 +184,9 @@ __device__ __forceinline__ float sum2<f16_t>(uint32_t w, float acc) {
 // Headroom of the lazy rescale, in log2 units: probabilities up to 2^8.
 constexpr float kRescaleSlack = 8.0f;
 
-template <typename T, int G, bool kBias, bool kVs, bool kSplit, int kMode, int kD>
+template <typename T, bool kBias, bool kVs, bool kSplit, int kMode, int kD, bool kExactP>
 __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
-  static_assert(kD == 128 || kD == 64, "head_dim 128, or 64 on table-less pages");
+  static_assert(kD == 128 || kD == 64, "head_dim 128 or 64");
   constexpr bool kDense = kMode == 1;
   constexpr bool kBig = kMode == 3;  // pages of 16 * 2^k tokens, k >= 1
   constexpr int kKRow = PfGeom<kD>::kKRow;
@@ -171,11 +196,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   constexpr int kDB = kD / 32;  // PV d-blocks (O accumulators)
   typedef typename Mma32<T>::v8 v8;
   typedef typename Mma32<T>::v4 v4;
-  constexpr int kPos = kPfRows / G;  // query positions per workgroup
+  const int G = p.G;
+  const int kPos = (unsigned)kPfRows / (unsigned)G;  // query positions per workgroup (rows past kPos * G idle)
   extern __shared__ __align__(16) unsigned char smem[];
   T* ks = reinterpret_cast<T*>(smem);                                                // [stage][64][kKRow]
   uint32_t* vts = reinterpret_cast<uint32_t*>(smem + (size_t)kPfStages * kKStage * 2);  // [stage][128][kVRowW]
   float* fbs = reinterpret_cast<float*>(vts + kPfStages * kVStage);                   // [stage][64] bias*log2(e)
+  float* fws = fbs + kPfStages * kPfKT;                                               // [stage][64] V weights (kExactP)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uniform(tid >> 6);
@@ -290,8 +317,9 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 
   // This lane's query row.
   const int frow = wave * 32 + col;
-  const int qi = qi_first + frow / G;
-  const int head = g * G + frow % G;
+  const int fpos = (unsigned)frow / (unsigned)G;
+  const int qi = qi_first + fpos;
+  const int head = g * G + frow - fpos * G;
   const int q_pos = ctx - C + qi;
   const bool row_ok = qi <= qi_last && q_pos >= 0;
 
@@ -450,7 +478,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   // Two register sets: the loads of tile t+3 go out in iteration t, one
   // iteration before their stage store, and land behind a whole iteration.
   v8 kreg[2][kKL], vreg[2][2];
-  float fw0[2] = {1.0f, 1.0f}, fw1[2] = {1.0f, 1.0f}, fb_r[2] = {0.0f, 0.0f};
+  float fw0[2] = {1.0f, 1.0f}, fw1[2] = {1.0f, 1.0f}, fb_r[2] = {0.0f, 0.0f}, fk_r[2] = {0.0f, 0.0f};
   auto issue = [&](int tile, const TileIds& tid_s, int set) {
     const int t0 = t_begin + tile * kstep;
     int64_t k_at;
@@ -467,18 +495,22 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       const auto vrs = span_rsrc(vpool, v_at, v_bytes);
       vreg[set][0] = __builtin_bit_cast(v8, __builtin_amdgcn_raw_buffer_load_b128(vrs, (int)voff0, 0, 0));
       vreg[set][1] = __builtin_bit_cast(v8, __builtin_amdgcn_raw_buffer_load_b128(vrs, (int)voff1, 0, 0));
-      if (kVs) {
+      if (kVs && !kExactP) {
         const int o = (t0 + vkey_off) * 4;
         fw0[set] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fw_rsrc, o, 0, 0));
         fw1[set] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fw1_rsrc, o, 0, 0));
       }
     }
+    if (kVs && kExactP)
+      fk_r[set] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fw_rsrc, (t0 + (tid & 63)) * 4, 0, 0));
     if (kBias)
       fb_r[set] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fb_rsrc, (t0 + (tid & 63)) * 4, 0, 0));
   };
   // V-fog: V rows are scaled by their fog weights here, rounded to T, as the
   // reference scales V before its product (v * fog_weights), so the
   // probabilities stay unscaled and the softmax sum can be taken from them.
+  // (kExactP: V stays as it is and the fp32 probabilities take the weights.)
+  constexpr bool kScaleV = kVs && !kExactP;
   auto store = [&](int stage, int set) {
     T* kd = ks + stage * kKStage + 8 * kc;
 #pragma unroll
@@ -487,10 +519,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       uint32_t* vd = vts + stage * kVStage + 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        vd[(8 * kc + e) * kVRowW] = kVs ? pack2<T>(to_f32(vreg[set][0][e]) * fw0[set], to_f32(vreg[set][1][e]) * fw1[set])
+        vd[(8 * kc + e) * kVRowW] = kScaleV ? pack2<T>(to_f32(vreg[set][0][e]) * fw0[set], to_f32(vreg[set][1][e]) * fw1[set])
                                         : bits16(vreg[set][0][e]) | (bits16(vreg[set][1][e]) << 16);
     }
     if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
+    if (kVs && kExactP && tid < kPfKT) fws[stage * kPfKT + tid] = fk_r[set];
   };
 
   // Slice i of n (n >= 8) of store(): V^T word i for i < 8, then the K rows
@@ -499,7 +532,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   auto store_slice = [&](int stage, int i, int n, int set) {
     if (vload && i < 8) {
       uint32_t* vd = vts + stage * kVStage + 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
-      vd[(8 * kc + i) * kVRowW] = kVs ? pack2<T>(to_f32(vreg[set][0][i]) * fw0[set], to_f32(vreg[set][1][i]) * fw1[set])
+      vd[(8 * kc + i) * kVRowW] = kScaleV ? pack2<T>(to_f32(vreg[set][0][i]) * fw0[set], to_f32(vreg[set][1][i]) * fw1[set])
                                       : bits16(vreg[set][0][i]) | (bits16(vreg[set][1][i]) << 16);
     }
     if (i == n - 1) {
@@ -507,6 +540,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 #pragma unroll
       for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
       if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
+      if (kVs && kExactP && tid < kPfKT) fws[stage * kPfKT + tid] = fk_r[set];
     }
   };
   // S^T of the tile in a stage: lane (col, half) reads K row 32kb + col.
@@ -639,11 +673,25 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     };
     float ps0 = 0.0f, ps1 = 0.0f;  // the softmax sum, from p as rounded for PV
     u32x4 pb[4];                   // p as the PV B operand, two keys per dword
+    u32x4 pl[4];                   // kExactP: what pb's rounding left of p, likewise
+    const float* fwt = fws + st_cur * kPfKT + 8 * half;
     auto exp_pair = [&](int j) {   // keys 2j, 2j+1 of this lane's 32
       const int kb = j >> 3, v = 2 * (j & 7);
       const float y0 = sc(kb)[v], y1 = sc(kb)[v + 1];
-      const float p0 = __builtin_amdgcn_exp2f(kBias ? y0 - muse : fmaf(y0, c2, -muse));
-      const float p1 = __builtin_amdgcn_exp2f(kBias ? y1 - muse : fmaf(y1, c2, -muse));
+      float p0 = __builtin_amdgcn_exp2f(kBias ? y0 - muse : fmaf(y0, c2, -muse));
+      float p1 = __builtin_amdgcn_exp2f(kBias ? y1 - muse : fmaf(y1, c2, -muse));
+      if constexpr (kExactP) {
+        ps0 += p0;
+        ps1 += p1;
+        if (kVs) {
+          p0 *= fwt[32 * kb + 16 * (v >> 3) + (v & 7)];
+          p1 *= fwt[32 * kb + 16 * (v >> 3) + (v & 7) + 1];
+        }
+        const uint32_t hi = pack2<T>(p0, p1);
+        pb[j >> 2][j & 3] = hi;
+        pl[j >> 2][j & 3] = pack2<T>(p0 - unpack_lo<T>(hi), p1 - unpack_hi<T>(hi));
+        return;
+      }
       const uint32_t w = pack2<T>(p0, p1);
       pb[j >> 2][j & 3] = w;
       if (j & 1)
@@ -666,6 +714,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       } else {
         const int s = (i - kQ) / kDB, db = (i - kQ) % kDB;
         oacc[db] = Mma32<T>::mma(op[i % 3], __builtin_bit_cast(v8, pb[s]), oacc[db]);
+        if constexpr (kExactP) oacc[db] = Mma32<T>::mma(op[i % 3], __builtin_bit_cast(v8, pl[s]), oacc[db]);
       }
       if (i + 2 < kQ + kPV) op[(i + 2) % 3] = op_read(i + 2);
       if (i < kQ) {
@@ -714,7 +763,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 
   // Lane (col, half) holds row frow at d = 32*db + 8*(v/4) + 4*half + (v%4).
   const float l = l_half + __shfl_xor(l_half, 32);
-  if (!row_ok) return;
+  // (A row before position 0 saw no key: it stores zeros, or an empty partial.)
+  if (qi > qi_last) return;
   if (kSplit && part_out) {
     // Split partial: unnormalised O, the running max in natural-log units
     // (the softmax here is base 2) and the sum, merged by the combine kernel.
@@ -746,13 +796,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     }
 }
 
-template <typename T, int G, bool kBias, bool kVs, bool kSplit, int kMode = 0, int kD = 128>
+template <typename T, bool kBias, bool kVs, bool kSplit, int kMode, int kD, bool kExactP>
 int launch_one(const Params& p, dim3 grid, hipStream_t stream) {
   static bool lds_set[64] = {};  // per instance and device
-  constexpr size_t lds = PfGeom<kD>::kLdsBytes;
+  constexpr size_t lds = PfGeom<kD>::lds_bytes(kExactP);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  const void* fn = reinterpret_cast<const void*>(prefill_mfma_kernel<T, G, kBias, kVs, kSplit, kMode, kD>);
+  const void* fn = reinterpret_cast<const void*>(prefill_mfma_kernel<T, kBias, kVs, kSplit, kMode, kD, kExactP>);
   if (!lds_set[dev]) {
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
       set_error(KESSIE_ERR_HIP, "fog prefill (mfma): %zu bytes of LDS unavailable", lds);
@@ -760,29 +810,46 @@ int launch_one(const Params& p, dim3 grid, hipStream_t stream) {
     }
     lds_set[dev] = true;
   }
-  hipLaunchKernelGGL((prefill_mfma_kernel<T, G, kBias, kVs, kSplit, kMode, kD>), grid, dim3(kPfThreads), lds, stream,
+  hipLaunchKernelGGL((prefill_mfma_kernel<T, kBias, kVs, kSplit, kMode, kD, kExactP>), grid, dim3(kPfThreads), lds, stream,
                      p);
   return check_launch("fog prefill (mfma)");
 }
 
-template <typename T, int G, bool kSplit, int kMode = 0>
+template <typename T, bool kSplit, int kMode, int kD, bool kExactP>
 int launch_fog(const Params& p, dim3 grid, hipStream_t stream) {
-  if (p.bias)
-    return p.vscale ? launch_one<T, G, true, true, kSplit, kMode>(p, grid, stream)
-                    : launch_one<T, G, true, false, kSplit, kMode>(p, grid, stream);
-  return p.vscale ? launch_one<T, G, false, true, kSplit, kMode>(p, grid, stream)
-                  : launch_one<T, G, false, false, kSplit, kMode>(p, grid, stream);
+  if constexpr (kMode != 1) {  // (the dense launchers have no bias)
+    if (p.bias)
+      return p.vscale ? launch_one<T, true, true, kSplit, kMode, kD, kExactP>(p, grid, stream)
+                      : launch_one<T, true, false, kSplit, kMode, kD, kExactP>(p, grid, stream);
+  }
+  return p.vscale ? launch_one<T, false, true, kSplit, kMode, kD, kExactP>(p, grid, stream)
+                  : launch_one<T, false, false, kSplit, kMode, kD, kExactP>(p, grid, stream);
 }
 
 // The split and longest-first instances are separate: the plain loop keeps the
 // register allocation it was tuned with (folding either into it cost the
 // V-fog long-context shape 1-6 %).
-template <typename T, int G>
-int launch_split(const Params& p, dim3 grid, hipStream_t stream) {
-  if (p.page_size > 16)  // pages of 16 * 2^k tokens (in query order)
-    return p.direct_out ? launch_fog<T, G, false, 3>(p, grid, stream) : launch_fog<T, G, true, 3>(p, grid, stream);
-  if (!p.direct_out) return launch_fog<T, G, true>(p, grid, stream);
-  return p.reverse_q ? launch_fog<T, G, false, 2>(p, grid, stream) : launch_fog<T, G, false>(p, grid, stream);
+template <typename T, int kD, bool kExactP>
+int launch_mode(const Params& p, dim3 grid, hipStream_t stream) {
+  if (p.page_table == nullptr)  // table-less pages (dense launchers): G 1, no bias
+    return p.num_splits > 1 ? launch_fog<T, true, 1, kD, kExactP>(p, grid, stream)
+                            : launch_fog<T, false, 1, kD, kExactP>(p, grid, stream);
+  if constexpr (kD == 128 || kExactP) {  // (head_dim 64 on pages: kExactP only)
+    if (p.page_size > 16)  // pages of 16 * 2^k tokens (in query order)
+      return p.direct_out ? launch_fog<T, false, 3, kD, kExactP>(p, grid, stream)
+                          : launch_fog<T, true, 3, kD, kExactP>(p, grid, stream);
+    if (!p.direct_out) return launch_fog<T, true, 0, kD, kExactP>(p, grid, stream);
+    return p.reverse_q ? launch_fog<T, false, 2, kD, kExactP>(p, grid, stream)
+                       : launch_fog<T, false, 0, kD, kExactP>(p, grid, stream);
+  }
+  set_error(KESSIE_ERR_UNSUPPORTED, "fog prefill (mfma): head_dim %d", p.D);
+  return KESSIE_ERR_UNSUPPORTED;
+}
+
+// Shapes whose probabilities are kept to fp32 precision (kernel header): paged
+// head_dim 64 and GQA ratios that are no power of two.
+bool prefill_exact_p(const Params& p) {
+  return p.page_table != nullptr && (p.D == 64 || (p.G & (p.G - 1)) != 0);
 }
 
 template <typename T>
@@ -790,33 +857,13 @@ int launch_prefill(Params& p, hipStream_t stream) {
   const int kpos = kPfRows / p.G;
   // Varlen: the live (sequence, query tile) pairs are numbered along x.
   dim3 grid(div_up(p.C, kpos) * p.Hkv * (p.q_start ? p.B : 1), p.q_start ? 1 : p.B, max(p.num_splits, 1));
-  // (The dense split instance numbers its (tile, split) units along x.)
-  if (p.page_table == nullptr) {  // table-less pages (dense launchers): G 1, no bias
-    if (p.num_splits > 1) {  // (tile, split) units along x (kernel header)
-      const int nq = div_up(p.C, kPfRows), t0 = p.split_q0 / kPfRows;
-      grid = dim3((unsigned)((t0 + (nq - t0) * p.num_splits) * p.Hkv), p.B, 1);
-      if (p.D == 64)
-        return p.vscale ? launch_one<T, 1, false, true, true, 1, 64>(p, grid, stream)
-                        : launch_one<T, 1, false, false, true, 1, 64>(p, grid, stream);
-      return p.vscale ? launch_one<T, 1, false, true, true, 1>(p, grid, stream)
-                      : launch_one<T, 1, false, false, true, 1>(p, grid, stream);
-    }
-    if (p.D == 64)
-      return p.vscale ? launch_one<T, 1, false, true, false, 1, 64>(p, grid, stream)
-                      : launch_one<T, 1, false, false, false, 1, 64>(p, grid, stream);
-    return p.vscale ? launch_one<T, 1, false, true, false, 1>(p, grid, stream)
-                    : launch_one<T, 1, false, false, false, 1>(p, grid, stream);
+  if (p.page_table == nullptr && p.num_splits > 1) {  // dense split: (tile, split) units along x (kernel header)
+    const int nq = div_up(p.C, kPfRows), t0 = p.split_q0 / kPfRows;
+    grid = dim3((unsigned)((t0 + (nq - t0) * p.num_splits) * p.Hkv), p.B, 1);
   }
-  switch (p.G) {
-    case 1: return launch_split<T, 1>(p, grid, stream);
-    case 2: return launch_split<T, 2>(p, grid, stream);
-    case 4: return launch_split<T, 4>(p, grid, stream);
-    case 8: return launch_split<T, 8>(p, grid, stream);
-    case 16: return launch_split<T, 16>(p, grid, stream);
-    default:
-      set_error(KESSIE_ERR_UNSUPPORTED, "fog prefill (mfma): GQA ratio %d", p.G);
-      return KESSIE_ERR_UNSUPPORTED;
-  }
+  if (prefill_exact_p(p))
+    return p.D == 64 ? launch_mode<T, 64, true>(p, grid, stream) : launch_mode<T, 128, true>(p, grid, stream);
+  return p.D == 64 ? launch_mode<T, 64, false>(p, grid, stream) : launch_mode<T, 128, false>(p, grid, stream);
 }
 
 }  // namespace
@@ -824,15 +871,14 @@ int launch_prefill(Params& p, hipStream_t stream) {
 bool prefill_mfma_ok(const Params& p, int dtype) {
   if (env_int("KESSIE_FORCE_GENERIC", 0)) return false;
   if (dtype != KESSIE_DTYPE_BF16 && dtype != KESSIE_DTYPE_F16) return false;
-  // Head_dim 64 only on table-less pages (the dense launchers).
-  if (!(p.D == 128 || (p.D == 64 && p.page_table == nullptr))) return false;
+  if (p.D != 128 && p.D != 64) return false;
   // Pages of 16 * 2^k tokens (table-less pages: 16), block ids (page << k) below 2^31.
   if (p.page_size < 16 || (p.page_size & (p.page_size - 1)) != 0 || (p.page_table == nullptr && p.page_size != 16))
     return false;
   if (((int64_t)p.num_pages << (__builtin_ctz((unsigned)p.page_size) - 4)) >= (int64_t)1 << 31) return false;
   // Table-less pages: instantiated for the dense launchers' form only.
   if (p.page_table == nullptr && (p.dense_ppb <= 0 || p.G != 1 || p.bias)) return false;
-  if (!(p.G == 1 || p.G == 2 || p.G == 4 || p.G == 8 || p.G == 16)) return false;
+  if (p.G < 1 || p.G > 16) return false;
   if (!(p.sm_scale > 0.0f)) return false;
   if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v) || !aligned16(p.out)) return false;
   if (p.page_stride % 8 || p.tok_stride % 8 || p.head_stride % 8) return false;

@@ -530,11 +530,11 @@ class KeSSieAttentionImpl:
             qs = meta.query_start_loc[lo:hi + 1]
             if qs.dtype != torch.int32:
                 qs = qs.to(torch.int32)
-            if ops.fog_prefill_varlen(q[s0:s1], qs, max(qsl[i + 1] - qsl[i] for i in prefill), kv_cache,
-                                      table[lo:hi], lens[lo:hi], kv_len,
-                                      fog_bias=None if bias is None else bias[lo:hi], window=self.window,
-                                      causal=True, sm_scale=self.scale, layout=layout, out=out[s0:s1],
-                                      stream=sp):
+            if ops.fog_prefill_batch(q[s0:s1], qs, max(qsl[i + 1] - qsl[i] for i in prefill), kv_cache,
+                                     table[lo:hi], lens[lo:hi], kv_len,
+                                     fog_bias=None if bias is None else bias[lo:hi], window=self.window,
+                                     causal=True, sm_scale=self.scale, layout=layout, out=out[s0:s1],
+                                     stream=sp):
                 prefill = []
         for i in prefill:
             s, e = qsl[i], qsl[i + 1]

@@ -1,0 +1,82 @@
+"""GPU parity of chunked prefill on head_dim 64 and on GQA ratios that are no
+power of two: MFMA instances whose probabilities keep fp32 precision.
+
+Tolerance: the kernel's own error is that of fp32 sums (2e-5 of the result's
+norm, far above 2^-16 per probability), so the distance from the oracle is that
+of rounding the oracle's result to the type, and no more."""
+import pytest
+import torch
+
+from oracle.attention import paged_prefill_ref
+from oracle.fog import fog_bias
+from tests.inputs import decode_case, gen, randn
+
+pytestmark = pytest.mark.gpu
+
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+def _close(out, ref, dtype):
+    err = (out.double().cpu() - ref.double()).norm()
+    rounding = (ref.to(dtype).double() - ref.double()).norm()
+    assert err <= 1.02 * rounding + 2e-5 * ref.double().norm(), f"error {err:.3e}, rounding alone {rounding:.3e}"
+
+
+def _fog(kind, b, ctx, dev):
+    vs = torch.rand(b, ctx, generator=gen(dev, 5), device=dev) if kind in ("vscale", "both") else None
+    bias = fog_bias(ctx, 0.5, 0.5, {3, 17}, 0.1).to(dev).repeat(b, 1) if kind in ("bias", "both") else None
+    return vs, bias
+
+
+@pytest.mark.parametrize("hq,hkv,d,c,ctxs,page,window,fog,dt,splits", [
+    (32, 8, 64, 70, [200, 70], 16, 0, "vscale", "bf16", 0),    # a query tile and six rows
+    (8, 8, 64, 256, [256], 16, 0, "none", "fp16", 0),          # one query tile, fresh prompt
+    (32, 8, 64, 1, [1, 64, 65], 16, 0, "both", "bf16", 0),     # one query, edges of a key tile
+    (32, 4, 64, 33, [1500], 32, 100, "bias", "fp16", 3),       # larger pages, window, key splits
+    (32, 8, 64, 1100, [1100], 16, 0, "bias", "bf16", 1),       # several rounds, longest tiles first
+    (24, 8, 128, 86, [300, 86], 16, 0, "vscale", "fp16", 0),   # GQA 3: 85 positions a workgroup
+    (40, 8, 128, 52, [900, 31], 16, 64, "both", "bf16", 2),    # GQA 5, splits, a chunk longer than its context
+    (28, 4, 64, 37, [400], 32, 0, "vscale", "fp16", 0),        # GQA 7, head_dim 64
+    (12, 1, 128, 22, [1000], 64, 0, "none", "bf16", 0),        # GQA 12: 21 positions a workgroup
+])
+def test_prefill_exact_p_shapes(dev, monkeypatch, hq, hkv, d, c, ctxs, page, window, fog, dt, splits):
+    from kessie_amd import ops
+
+    if splits:
+        monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
+    b, mx, dtype = len(ctxs), max(ctxs), DT[dt]
+    _, pool, table, lens = decode_case(b, hq, hkv, d, mx, page, dtype, dev, seed=7, ctx_lens=ctxs)
+    q = randn((b, c, hq, d), dtype, dev, 8)
+    vs, bias = _fog(fog, b, mx, dev)
+    out = torch.full_like(q, float("nan"))
+    ops.fog_prefill(q, pool, table, lens, mx, fog_vscale=vs, fog_bias=bias, window=window, out=out)
+    torch.cuda.synchronize()
+    for i, n in enumerate(ctxs):
+        live = max(0, c - n)  # queries before position 0 see no key: zeros
+        assert not out[i, :live].any()
+        ref = paged_prefill_ref(q[i:i + 1, live:].cpu(), pool.cpu(), table[i:i + 1].cpu(), lens[i:i + 1].cpu(),
+                                None if vs is None else vs[i:i + 1].cpu(),
+                                None if bias is None else bias[i:i + 1].cpu(), window)
+        _close(out[i:i + 1, live:], ref, dtype)
+
+
+@pytest.mark.parametrize("hq,hkv,d,page", [(32, 8, 64, 16), (24, 8, 128, 32), (32, 8, 128, 16)])
+def test_prefill_batch_matches_per_sequence(dev, monkeypatch, hq, hkv, d, page):
+    """One launch over ragged chunks equals the per-sequence launches bit for bit (one key split)."""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", "1")
+    chunks, ctxs = [90, 1, 33, 260], [200, 64, 33, 700]
+    _, pool, table, lens = decode_case(4, hq, hkv, d, max(ctxs), page, torch.bfloat16, dev, seed=17, ctx_lens=ctxs)
+    starts = [0, 90, 91, 124, 384]
+    qsl = torch.tensor(starts, dtype=torch.int32, device=dev)
+    q = randn((384, hq, d), torch.bfloat16, dev, 18)
+    bias = fog_bias(max(ctxs), 0.5, 0.5, {3}, 0.1).to(dev).repeat(4, 1)
+    out = torch.full_like(q, float("nan"))
+    listed = d == 128 and (hq // hkv) & (hq // hkv - 1) == 0
+    assert ops.fog_prefill_varlen(q, qsl, 260, pool, table, lens, max(ctxs), fog_bias=bias, out=out) == listed
+    assert ops.fog_prefill_batch(q, qsl, 260, pool, table, lens, max(ctxs), fog_bias=bias, out=out)
+    for i in range(4):
+        s, e = starts[i], starts[i + 1]
+        one = ops.fog_prefill(q[s:e][None], pool, table[i:i + 1], lens[i:i + 1], max(ctxs), fog_bias=bias[i:i + 1])
+        assert torch.equal(out[s:e], one[0]), i
