@@ -56,6 +56,8 @@
 //            store their output directly); 2 paged with query tiles longest first (a causal chunk
 //            that is most of its context and takes several grid rounds); 3
 //            paged with pages of 32, 64, ... tokens, read as 16-token blocks.
+#include <type_traits>
+
 #include "attn_common.h"
 
 namespace kessie {
@@ -74,9 +76,9 @@ struct PfGeom {
   static constexpr int kKRow = D + 8;            // K tile row stride (elements)
   static constexpr int kKStage = kPfKT * kKRow;  // elements per K stage
   static constexpr int kVStage = D * kVRowW;     // words per V^T stage
-  // K, V^T, bias; the exact-P instances also keep the tile's V weights.
+  // K, V^T, bias; the exact-P instances also keep the tile's V weights and their largest magnitude.
   static constexpr size_t lds_bytes(bool exact_p) {
-    return (size_t)kPfStages * (kKStage * 2 + kVStage * 4 + kPfKT * 4 * (exact_p ? 2 : 1));
+    return (size_t)kPfStages * (kKStage * 2 + kVStage * 4 + kPfKT * 4 * (exact_p ? 2 : 1) + (exact_p ? 4 : 0));
   }
 };
 constexpr float kLog2e = 1.4426950408889634f;
@@ -167,6 +169,20 @@ __device__ __forceinline__ float max_xor32(float x) {
   return max3(a, b, b);
 }
 
+// max over the wave's lanes, in every lane (DPP within the rows of 16).
+__device__ __forceinline__ float wave_max(float x) {
+  auto dpp = [](float v, auto ctrl) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  x = fmaxf(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // quad_perm 1,0,3,2
+  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // quad_perm 2,3,0,1
+  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+  auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l)); };
+  return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
+}
+
 // acc + lo + hi of two packed T values (one v_dot2 against (1, 1)).
 template <typename T>
 __device__ __forceinline__ float sum2(uint32_t w, float acc);
@@ -183,6 +199,13 @@ __device__ __forceinline__ float sum2<f16_t>(uint32_t w, float acc) {
 
 // Headroom of the lazy rescale, in log2 units: probabilities up to 2^8.
 constexpr float kRescaleSlack = 8.0f;
+// fp16 kExactP with V weights: p * w enters PV as fp16 operands, whose range
+// holds neither weights above 2^8 nor small ones to full precision.  The
+// exponentials' reference is therefore m_run + e_run, e_run an exponent of the
+// largest weight so far (within 2^kWRange of 1; raised when a tile's weights
+// exceed it by 2^kWSlack), which scales O and the softmax sum alike.
+constexpr int kWRange = 60;
+constexpr int kWSlack = 7;  // p * w < 2^(kRescaleSlack + kWSlack) = 2^15
 
 template <typename T, bool kBias, bool kVs, bool kSplit, int kMode, int kD, bool kExactP>
 __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
@@ -203,6 +226,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   uint32_t* vts = reinterpret_cast<uint32_t*>(smem + (size_t)kPfStages * kKStage * 2);  // [stage][128][kVRowW]
   float* fbs = reinterpret_cast<float*>(vts + kPfStages * kVStage);                   // [stage][64] bias*log2(e)
   float* fws = fbs + kPfStages * kPfKT;                                               // [stage][64] V weights (kExactP)
+  float* fwm = fws + kPfStages * kPfKT;                                               // [stage] their max magnitude
+  constexpr bool kWExp = kExactP && kVs && std::is_same<T, f16_t>::value;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uniform(tid >> 6);
@@ -511,6 +536,12 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   // probabilities stay unscaled and the softmax sum can be taken from them.
   // (kExactP: V stays as it is and the fp32 probabilities take the weights.)
   constexpr bool kScaleV = kVs && !kExactP;
+  auto store_weights = [&](int stage, int set) {
+    if (kVs && kExactP && tid < kPfKT) {  // wave 0
+      fws[stage * kPfKT + tid] = fk_r[set];
+      if constexpr (kWExp) fwm[stage] = wave_max(fabsf(fk_r[set]));
+    }
+  };
   auto store = [&](int stage, int set) {
     T* kd = ks + stage * kKStage + 8 * kc;
 #pragma unroll
@@ -523,7 +554,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
                                         : bits16(vreg[set][0][e]) | (bits16(vreg[set][1][e]) << 16);
     }
     if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
-    if (kVs && kExactP && tid < kPfKT) fws[stage * kPfKT + tid] = fk_r[set];
+    store_weights(stage, set);
   };
 
   // Slice i of n (n >= 8) of store(): V^T word i for i < 8, then the K rows
@@ -540,7 +571,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 #pragma unroll
       for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
       if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
-      if (kVs && kExactP && tid < kPfKT) fws[stage * kPfKT + tid] = fk_r[set];
+      store_weights(stage, set);
     }
   };
   // S^T of the tile in a stage: lane (col, half) reads K row 32kb + col.
@@ -563,6 +594,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 #pragma unroll
   for (int i = 0; i < kDB; ++i) oacc[i] = f32x16{};
   float m_run = kNegInf, l_half = 0.0f;
+  float e_run = -(float)kWRange;  // (kWExp)
   const float c2 = p.sm_scale * kLog2e;
 
   // Tiles whose 64 keys all lie in [lo, hi) and are visible to every row of
@@ -647,8 +679,15 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     // kRescaleSlack (log2 units); until then p = 2^(y - m_run) <= 2^kRescaleSlack,
     // as exact in T as any p <= 1, and the O accumulators are left alone.
     const float mnew = mloc > m_run + kRescaleSlack ? mloc : m_run;
-    const float muse = mnew == kNegInf ? 0.0f : mnew;
-    const float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
+    float muse = mnew == kNegInf ? 0.0f : mnew;
+    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
+    if constexpr (kWExp) {
+      const int we = ((int)(__builtin_bit_cast(uint32_t, fwm[st_cur]) >> 23) & 255) - 127;  // floor(log2), uniform
+      const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
+      alpha *= __builtin_amdgcn_exp2f(e_run - e_new);
+      muse += e_new;
+      e_run = e_new;
+    }
     // (Rescaled before the exponentials, so that they, the next scores and PV
     // form one branch-free region.)
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
@@ -778,7 +817,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         *reinterpret_cast<f32x4*>(dst + 32 * db + 8 * vq) =
             f32x4{oacc[db][4 * vq], oacc[db][4 * vq + 1], oacc[db][4 * vq + 2], oacc[db][4 * vq + 3]};
     if (half == 0) {
-      p.ws_m[r] = m_run == kNegInf ? kNegInf : m_run * kLn2;
+      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m_run + e_run : m_run) * kLn2;
       p.ws_l[r] = l;
     }
     return;

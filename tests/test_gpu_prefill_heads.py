@@ -80,3 +80,20 @@ def test_prefill_batch_matches_per_sequence(dev, monkeypatch, hq, hkv, d, page):
         s, e = starts[i], starts[i + 1]
         one = ops.fog_prefill(q[s:e][None], pool, table[i:i + 1], lens[i:i + 1], max(ctxs), fog_bias=bias[i:i + 1])
         assert torch.equal(out[s:e], one[0]), i
+
+
+@pytest.mark.parametrize("hq,hkv,d,splits", [(8, 2, 64, 1), (8, 2, 64, 3), (6, 2, 128, 1)])
+@pytest.mark.parametrize("lo,hi,vmul", [(1e4, 1e4, 1.0), (1e-6, 1e-6, 1e3), (1e-6, 1e4, 1.0), (-900.0, 900.0, 1.0)])
+def test_prefill_fp16_weights_of_any_magnitude(dev, monkeypatch, hq, hkv, d, splits, lo, hi, vmul):
+    """V weights far from 1 (constant, or rising or changing sign along the context): p * w leaves fp16's range."""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
+    _, pool, table, lens = decode_case(1, hq, hkv, d, 500, 16, torch.float16, dev, seed=9, ctx_lens=[500])
+    pool = pool * vmul
+    q = randn((1, 90, hq, d), torch.float16, dev, 10) / vmul
+    ramp = torch.linspace(0, 1, 500, device=dev)
+    w = (lo + (hi - lo) * ramp if lo * hi < 0 else lo * (hi / lo) ** ramp).float().view(1, -1)
+    out = ops.fog_prefill(q, pool, table, lens, 500, fog_vscale=w)
+    ref = paged_prefill_ref(q.cpu(), pool.cpu(), table.cpu(), lens.cpu(), w.cpu(), None, 0)
+    _close(out, ref, torch.float16)
