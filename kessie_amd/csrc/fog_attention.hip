@@ -2328,19 +2328,25 @@ static void dense_fp16(const void* Q, const void* K, const void* V, void* O, con
     return;
   }
   // head_dim 128 or 64: the MFMA prefill kernel, reading the dense tensors as
-  // table-less 16-token pages (page b*H*N/16 + j = tokens 16j..16j+15 of every
-  // head of sequence b, heads N*D apart; H*N a multiple of 16 keeps sequences
-  // on whole pages, and the kernel reads no token past N).  Key splits
-  // (partials merged by the combine kernel) when the grid alone would leave
-  // CUs idle, in the library's per-stream buffer (these launchers take no
-  // workspace); without one, a single split.
-  const int64_t dense_pages = (int64_t)B * H * N / 16;
-  if (((int64_t)H * N) % 16 == 0 && dense_pages <= INT_MAX) {
-    Params m = p;
-    m.page_size = 16;
-    m.page_stride = 16 * (int64_t)D;
-    m.num_pages = (int)dense_pages;
-    m.dense_ppb = (int)(((int64_t)H * N) / 16);
+  // table-less 16-token pages (tokens 16j..16j+15 of every head, heads N*D
+  // apart; the kernel reads no token past N).  Key splits (partials merged by
+  // the combine kernel) when the grid alone would leave CUs idle, in the
+  // library's per-stream buffer (these launchers take no workspace); without
+  // one, a single split.  H*N a multiple of 16: probabilities rounded for PV.
+  // Other sizes: probabilities to fp32 precision, as on the fp32 VALU kernel
+  // that took them before (B=2, H=8, N=1,537, D=64, window 1,024: 722 us
+  // there, 39 us here).
+  const bool ragged = ((int64_t)H * N) % 16 != 0;
+  // Testing switch: KESSIE_REQUIRE_MFMA=1 makes a shape that is not on the
+  // rounded-probability route an error (the tests use it to show which route
+  // ran).
+  const bool require = env_int("KESSIE_REQUIRE_MFMA", 0) != 0;
+  Params m = p;
+  m.page_size = 16;
+  m.page_stride = 16 * (int64_t)D;
+  m.num_pages = div_up(N, 16);
+  m.dense_exact_p = ragged ? 1 : 0;
+  if (!(require && ragged)) {
     if (prefill_mfma_ok(m, KESSIE_DTYPE_F16)) {
       const hipStream_t s = as_stream(stream);
       int split_q0 = 0;
@@ -2365,11 +2371,9 @@ static void dense_fp16(const void* Q, const void* K, const void* V, void* O, con
       return;
     }
   }
-  // Testing switch: KESSIE_REQUIRE_MFMA=1 makes a shape that would fall back
-  // to the generic kernel an error instead (the tests use it to show which
-  // route ran).
-  if (env_int("KESSIE_REQUIRE_MFMA", 0)) {
-    set_error(KESSIE_ERR_UNSUPPORTED, "dense attention: B=%d H=%d N=%d D=%d runs on the generic kernel", B, H, N, D);
+  if (require) {
+    set_error(KESSIE_ERR_UNSUPPORTED, "dense attention: B=%d H=%d N=%d D=%d runs at the generic kernel's precision", B,
+              H, N, D);
     return;
   }
   launch_generic<f16_t>(p, as_stream(stream));

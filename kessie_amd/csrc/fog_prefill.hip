@@ -42,14 +42,18 @@
 //            kernel (attn_generic_kernel), which these shapes would otherwise
 //            take: 2,048 queries on 32,768 tokens at head_dim 64 49.3 ms there,
 //            0.96 ms (557 TFLOP/s) here; on 16,384 at 24 q / 8 kv heads of 128
-//            44.2 against 0.89 ms;
+//            44.2 against 0.89 ms.  Dense tensors whose H * N is no multiple of
+//            16 take it too (B=2, H=8, N=1,537, D=64, window 1,024: 722 us
+//            there, 39 us here; B=4, H=12, N=1,001, D=128, causal fog 2,035
+//            and 99 us);
 //   kSplit   grid z splits each query tile's key tiles (split s takes tiles
 //            s, s + S, ...); every split stores unnormalised partials (O,
 //            max, sum) merged by the combine kernel -- used when the chunks
 //            alone would leave CUs idle;
 //   q_start  varlen batch: x / Hkv numbers the live (sequence, query tile)
 //            pairs, each chunk's queries packed at query_start_loc;
-//   kMode    0 paged; 1 table-less pages (page b * dense_ppb + j) for the
+//   kMode    0 paged; 1 table-less pages (page j of a sequence: its tokens
+//            16j .. 16j + 15, any N) for the
 //            reference's dense [B][H][N][D] launchers, query tiles longest
 //            first (split: only the tiles from split_q0 on, S units each,
 //            numbered along x split-major with the unsplit tiles, which
@@ -379,7 +383,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   auto krow = [&](int r) { return kD == 128 ? 16 * kslot + rr + 8 * r : rr; };  // K key of the tile
   auto krow_lds = [&](int r) { return (krow(r) & 32) | swap23(krow(r) & 31); };  // its LDS row
   const int32_t* table = kDense ? nullptr : p.page_table + (int64_t)b * p.table_stride;
-  const int dense0 = kDense ? b * p.dense_ppb : 0;  // table-less pages: sequence b's first
   const bool vload = kD == 128 || wave < 4;
   const int vkey_off = 2 * kp;  // this thread's first V key in a tile
 
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     for (int j = 0; j < 4; ++j) {
       const bool in = tile < n_tiles && pg0 + j < n_tab;
       if constexpr (kDense) {
-        ids[j] = in ? dense0 + pg0 + j : -1;
+        ids[j] = in ? pg0 + j : -1;
       } else if constexpr (kBig) {
         const int e = table[min(pg0 + j, n_tab - 1) >> psh];
         ids[j] = in && (uint32_t)e < (uint32_t)p.num_pages ? (e << psh) | ((pg0 + j) & pmask) : -1;
@@ -443,7 +446,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     }
     r.ids = fetch_ids(tile);
     if constexpr (kDense) {
-      r.own = tile < n_tiles && pg0 + kslot < n_tab ? dense0 + pg0 + kslot : -1;
+      r.own = tile < n_tiles && pg0 + kslot < n_tab ? pg0 + kslot : -1;
     } else if constexpr (kBig) {
       const int j = pg0 + kslot;
       const int e = table[min(j, n_tab - 1) >> psh];
@@ -463,8 +466,10 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   constexpr int kKL = kD == 128 ? 2 : 1;  // K rows loaded per thread per tile
   const int ts_b = (int)p.tok_stride * (int)sizeof(T);
   constexpr int kRowB = kD * (int)sizeof(T);
-  const char* kpool = static_cast<const char*>(p.k) + (int64_t)g * p.head_stride * (int64_t)sizeof(T);
-  const char* vpool = static_cast<const char*>(p.v) + (int64_t)g * p.head_stride * (int64_t)sizeof(T);
+  // (Dense: page ids count from the sequence's own start, as wide as a query's.)
+  const int64_t head_b = ((int64_t)g * p.head_stride + (kDense ? (int64_t)b * p.q_bs : 0)) * (int64_t)sizeof(T);
+  const char* kpool = static_cast<const char*>(p.k) + head_b;
+  const char* vpool = static_cast<const char*>(p.v) + head_b;
   uint32_t koff[kKL];
 #pragma unroll
   for (int r = 0; r < kKL; ++r) koff[r] = (uint32_t)((krow(r) & 15) * ts_b + 16 * kc);
@@ -870,9 +875,11 @@ int launch_fog(const Params& p, dim3 grid, hipStream_t stream) {
 // V-fog long-context shape 1-6 %).
 template <typename T, int kD, bool kExactP>
 int launch_mode(const Params& p, dim3 grid, hipStream_t stream) {
-  if (p.page_table == nullptr)  // table-less pages (dense launchers): G 1, no bias
-    return p.num_splits > 1 ? launch_fog<T, true, 1, kD, kExactP>(p, grid, stream)
-                            : launch_fog<T, false, 1, kD, kExactP>(p, grid, stream);
+  if constexpr (__is_same(T, f16_t)) {
+    if (p.page_table == nullptr)  // table-less pages (dense launchers): fp16, G 1, no bias
+      return p.num_splits > 1 ? launch_fog<T, true, 1, kD, kExactP>(p, grid, stream)
+                              : launch_fog<T, false, 1, kD, kExactP>(p, grid, stream);
+  }
   if constexpr (kD == 128 || kExactP) {  // (head_dim 64 on pages: kExactP only)
     if (p.page_size > 16)  // pages of 16 * 2^k tokens (in query order)
       return p.direct_out ? launch_fog<T, false, 3, kD, kExactP>(p, grid, stream)
@@ -886,9 +893,10 @@ int launch_mode(const Params& p, dim3 grid, hipStream_t stream) {
 }
 
 // Shapes whose probabilities are kept to fp32 precision (kernel header): paged
-// head_dim 64 and GQA ratios that are no power of two.
+// head_dim 64, GQA ratios that are no power of two, and the dense tensors that
+// ask for it.
 bool prefill_exact_p(const Params& p) {
-  return p.page_table != nullptr && (p.D == 64 || (p.G & (p.G - 1)) != 0);
+  return p.page_table != nullptr ? p.D == 64 || (p.G & (p.G - 1)) != 0 : p.dense_exact_p != 0;
 }
 
 template <typename T>
@@ -916,7 +924,7 @@ bool prefill_mfma_ok(const Params& p, int dtype) {
     return false;
   if (((int64_t)p.num_pages << (__builtin_ctz((unsigned)p.page_size) - 4)) >= (int64_t)1 << 31) return false;
   // Table-less pages: instantiated for the dense launchers' form only.
-  if (p.page_table == nullptr && (p.dense_ppb <= 0 || p.G != 1 || p.bias)) return false;
+  if (p.page_table == nullptr && (dtype != KESSIE_DTYPE_F16 || p.G != 1 || p.bias)) return false;
   if (p.G < 1 || p.G > 16) return false;
   if (!(p.sm_scale > 0.0f)) return false;
   if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v) || !aligned16(p.out)) return false;
