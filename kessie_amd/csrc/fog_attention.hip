@@ -12,13 +12,14 @@
 //
 // Kernels:
 //   decode_mfma   bf16/f16 (fp32: decode_mfma_f32 on v_mfma_f32_16x16x4_f32,
-//                 same decomposition), head_dim 128, pages of 16 * 2^k tokens
+//                 same decomposition), head_dim 128 (bf16/f16 also 64), GQA
+//                 ratios up to 16 (fp32: powers of two), pages of 16 * 2^k tokens
 //                 (read as 16-token blocks).  One workgroup =
 //                 one (sequence, split) x 2 kv heads, one wave per kv head; a
-//                 wave streams its kv head's 256-byte K and V rows of every
+//                 wave streams its kv head's K and V rows of every
 //                 page in its split with 16-byte loads (register prefetch of
 //                 PREF pages); QK^T and PV both on MFMA (P in the input
-//                 dtype, accumulation in fp32), V transposed through LDS.
+//                 dtype, or as two operands of it, accumulation in fp32), V transposed through LDS.
 //   attn_generic  any dtype / head_dim <= 256 / page size / GQA ratio: K and
 //                 V tiles staged in LDS as fp32, one workgroup per
 //                 (row tile, kv head, sequence, split).  Serves the shapes the
@@ -32,6 +33,7 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -723,7 +725,8 @@ void launch_combine(const Params& p, int64_t rows, hipStream_t s) {
 
 
 // ---------------------------------------------------------------------------
-// MFMA decode (bf16 / f16, head_dim 128, pages of 16 * 2^k tokens)
+// MFMA decode (bf16 / f16, head_dim 128 or 64, pages of 16 * 2^k tokens).
+// Described for head_dim 128; 64 halves the rows and keeps the split.
 //
 // One workgroup = (split of one sequence's pages) x kDecWaves kv heads, one
 // wave per kv head, no workgroup barriers.  Per page a wave:
@@ -745,7 +748,6 @@ void launch_combine(const Params& p, int64_t rows, hipStream_t s) {
 constexpr int kDecWaves = 2;     // kv heads (waves) per decode workgroup
 constexpr int kDecPref = 2;      // pages in flight per wave
 constexpr int kDecWgsPerCu = 4;  // 2 waves/SIMD x 4 SIMDs / kDecWaves: one round of the grid
-constexpr int kVRow = 128 + 8;  // LDS row stride of the V and Q tiles (elements)
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -788,11 +790,32 @@ __device__ __forceinline__ void wave_lds_sync() {
 // bit 1 the V-scale); each one read costs a register per prefetched page.
 constexpr int kFogBias = 1, kFogVs = 2;
 
-template <typename T, int G, int PREF, int W, int FOG>
+// GT 0: any GQA ratio up to 16 (p.G).  kExact: p * w enters PV as two operands
+// of T, the rounded value and what the rounding left (p to 2^-16 relative in
+// bf16, 2^-22 in fp16), for the shapes the fp32 VALU kernel served before:
+// head_dim 64 and GQA ratios that are no power of two.  The loop waits on K
+// and V, not on the extra MFMAs.  Steps on the VALU kernel and here: head_dim
+// 64, 16 sequences of 131,072 tokens (32 q / 8 kv) 6,880 and 763 us (5.6 TB/s),
+// 12 of 600-6,000 143 and 36; head_dim 128 at GQA 3, 8 of 13,000-65,536
+// 2,454 and 174 (6.3 TB/s).
+// In fp16 with V weights, p * w is held in range by an exponent of the largest
+// weight so far, e_run, which scales O, the softmax sum and the stored max
+// alike; it moves when a page's weights exceed it by 2^kWSlack.
+constexpr int kWRange = 60;
+constexpr int kWSlack = 7;
+
+template <typename T, int GT, int PREF, int W, int FOG, int D, bool kExact>
 // Two waves per SIMD (256 VGPRs; ~160 used with two pages of K and V in flight).
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_mfma_kernel(Params p) {
   typedef typename Mfma<T>::vec8 vec8;
   typedef typename Mfma<T>::vec4 vec4;
+  constexpr int kVRow = D + 8;   // LDS row stride of the V and Q tiles (elements)
+  constexpr int kKB = D / 32;    // K loads (and QK MFMAs) per page
+  constexpr int kCh = D / 8;     // 16-byte chunks of a row
+  constexpr int kVL = D / 32;    // V loads per page, 64 / kCh tokens each
+  constexpr int kBlk = D / 16;   // O^T blocks
+  constexpr bool kWExp = kExact && (FOG & kFogVs) != 0 && std::is_same<T, f16_t>::value;
+  const int G = GT ? GT : p.G;
   __shared__ __align__(16) T vtile_all[W][16 * kVRow];
   __shared__ __align__(16) T qtile_all[W][16 * kVRow];
   const int lane = threadIdx.x & 63;
@@ -838,7 +861,10 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int psh = __builtin_ctz((unsigned)p.page_size) - 4;
   const int pmask = (1 << psh) - 1;
   const int64_t koff = (int64_t)row * ts + 8 * grp;        // + 32*kb
-  const int64_t voff = (int64_t)(4 * grp) * ts + 8 * row;  // + i*ts
+  // V rows of this lane: head_dim 128 its own token quad (4 grp + i), chunk
+  // `row`; head_dim 64 tokens lane / 8 + 8 i, chunk lane % 8.
+  auto vtok = [&](int i) { return D == 128 ? 4 * grp + i : lane / kCh + (64 / kCh) * i; };
+  const int vch = lane & (kCh - 1);
 
   // B operand of S^T = K Q^T: the GQA group's query rows (column = head),
   // kept in this wave's LDS tile (zero rows past G) and read per page, which
@@ -846,7 +872,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   {
     const T* qrow = static_cast<const T*>(p.q) + (int64_t)b * p.q_bs + (int64_t)(g * G + row) * p.q_hs;
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < kKB; ++kb) {
       vec8 x;
       if (row < G) {
         x = *reinterpret_cast<const vec8*>(qrow + 32 * kb + 8 * grp);
@@ -859,12 +885,14 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     wave_lds_sync();
   }
 
-  f32x4 oacc[8];  // O^T[d = 16*blk + 4*grp + i][head = row]
+  f32x4 oacc[kBlk];  // O^T[d = 16*blk + 4*grp + i][head = row]
 #pragma unroll
-  for (int blk = 0; blk < 8; ++blk) oacc[blk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int blk = 0; blk < kBlk; ++blk) oacc[blk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = kNegInf, l_run = 0.0f;  // softmax state of head `row`
 
-  vec8 kreg[PREF][4], vreg[PREF][4];
+  float e_run = -(float)kWRange;          // (kWExp)
+
+  vec8 kreg[PREF][kKB], vreg[PREF][kVL];
   int pid_s[PREF];
   // Per-token fog values of the next page to compute, lane t (< 16) holding
   // token 16*lp + t (0 outside [lo, ctx)).  They are loaded when the previous
@@ -891,10 +919,11 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       // Non-temporal: each K/V byte is read once per launch (measured 9 % faster
       // than plain loads for this access pattern).
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < kKB; ++kb)
         kreg[st][kb] = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(kp + koff + 32 * kb));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) vreg[st][i] = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(vp + voff + i * ts));
+      for (int i = 0; i < kVL; ++i)
+        vreg[st][i] = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(vp + (int64_t)vtok(i) * ts + 8 * vch));
     }
   };
 
@@ -919,7 +948,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       // Scores: lane (grp, row) holds head `row`, tokens t_page + 4*grp + i.
       f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int kb = 0; kb < kKB; ++kb) {
         const vec8 qv = *reinterpret_cast<const vec8*>(qtile + row * kVRow + 32 * kb + 8 * grp);
         acc = Mfma<T>::mma32(kreg[st][kb], qv, acc);
       }
@@ -936,12 +965,22 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
       mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
       const float mnew = fmaxf(m_run, mloc);
-      const float alpha = (m_run == kNegInf) ? 0.0f : __expf(m_run - mnew);
+      float alpha = (m_run == kNegInf) ? 0.0f : __expf(m_run - mnew);
+      float wsc = 1.0f;  // 2^-e_run
+      if constexpr (kWExp) {
+        const float wm = row_max16(fabsf(fv_cur));  // lanes 0..15 hold the page's weights
+        const int we = ((int)(__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wm)) >> 23) & 255) - 127;
+        const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
+        alpha *= __builtin_amdgcn_exp2f(e_run - e_new);
+        wsc = __builtin_amdgcn_exp2f(-e_new);
+        e_run = e_new;
+      }
       float pr[4];
       float psum = 0.0f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         pr[i] = (sc[i] == kNegInf) ? 0.0f : __expf(sc[i] - mnew);
+        if constexpr (kWExp) pr[i] *= wsc;
         psum += pr[i];
       }
       psum += __shfl_xor(psum, 16);
@@ -954,13 +993,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       }
       if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
-        for (int blk = 0; blk < 8; ++blk) oacc[blk] *= alpha;
+        for (int blk = 0; blk < kBlk; ++blk) oacc[blk] *= alpha;
       }
-      // V rows of this lane's token quad -> LDS tile (masked tokens as zeros).
+      // This lane's V rows -> LDS tile (masked tokens as zeros).
       if (!full) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = t_page + 4 * grp + i;
+        for (int i = 0; i < kVL; ++i) {
+          const int t = t_page + vtok(i);
           if (!(t >= lo && t < ctx)) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) vreg[st][i][e] = static_cast<T>(0.0f);
@@ -969,17 +1008,21 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       }
       wave_lds_sync();  // the previous page's transposed reads are done
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<vec8*>(vtile + (4 * grp + i) * kVRow + 8 * row) = vreg[st][i];
+      for (int i = 0; i < kVL; ++i) *reinterpret_cast<vec8*>(vtile + vtok(i) * kVRow + 8 * vch) = vreg[st][i];
       wave_lds_sync();
-      vec4 pb;
+      vec4 pb, pl;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pb[i] = static_cast<T>(pr[i]);
+      for (int i = 0; i < 4; ++i) {
+        pb[i] = static_cast<T>(pr[i]);
+        if constexpr (kExact) pl[i] = static_cast<T>(pr[i] - static_cast<float>(pb[i]));
+      }
 #pragma unroll
-      for (int blk = 0; blk < 8; ++blk) {
+      for (int blk = 0; blk < kBlk; ++blk) {
         vec4 va;
 #pragma unroll
         for (int i = 0; i < 4; ++i) va[i] = vtile[(4 * grp + i) * kVRow + 16 * blk + row];
         oacc[blk] = Mfma<T>::mma16(va, pb, oacc[blk]);
+        if constexpr (kExact) oacc[blk] = Mfma<T>::mma16(va, pl, oacc[blk]);
       }
       if (FOG && lp + 1 < p1) load_fog(lp + 1);
       if (lp + PREF < p1) issue(st, lp + PREF);
@@ -993,7 +1036,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     const float il = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     T* dst = static_cast<T*>(p.out) + (int64_t)b * p.o_bs + (int64_t)head * p.o_hs + 4 * grp;
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk) {
+    for (int blk = 0; blk < kBlk; ++blk) {
       vec4 ov;
 #pragma unroll
       for (int i = 0; i < 4; ++i) ov[i] = from_f32<T>(oacc[blk][i] * il);
@@ -1001,11 +1044,11 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   } else {
     const int64_t slot = p.balanced ? (int64_t)head * p.units + unit : row_id(p, b, 0, head) * S + split;
-    float* dst = p.ws_o + slot * 128 + 4 * grp;
+    float* dst = p.ws_o + slot * D + 4 * grp;
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk];
+    for (int blk = 0; blk < kBlk; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk];
     if (grp == 0) {
-      p.ws_m[slot] = m_run;
+      p.ws_m[slot] = kWExp ? m_run + e_run * 0.6931471805599453f : m_run;
       p.ws_l[slot] = l_run;
     }
   }
@@ -1354,21 +1397,25 @@ int launch_generic(Params& p, hipStream_t stream) {
   return KESSIE_OK;
 }
 
-template <typename T, int G>
+// PREF pages in flight: head_dim 64 pages hold half the bytes, so twice as many.
+template <typename T, int GT, int FOG, int D, bool kExact>
+void launch_decode_one(const Params& p, hipStream_t stream) {
+  constexpr int kPref = kDecPref * 128 / D;
+  hipLaunchKernelGGL((decode_mfma_kernel<T, GT, kPref, kDecWaves, FOG, D, kExact>), decode_grid(p), dim3(kDecWaves * 64), 0,
+                     stream, p);
+}
+
+template <typename T, int GT, int D = 128, bool kExact = false>
 int launch_decode_mfma(Params& p, hipStream_t stream) {
   // Two kv heads per workgroup, two pages in flight per wave, two waves per
   // SIMD (measured at batch 16, 128K context: 1.308 ms against 1.314 ms with
   // four pages in flight -- which also cost one sequence 3-9 % -- and 1.398 ms
   // with two pages at three waves per SIMD).
-  const dim3 grid = decode_grid(p);
-  const int fog = (p.bias ? kFogBias : 0) | (p.vscale ? kFogVs : 0);
-  const dim3 block(kDecWaves * 64);
-  switch (fog) {
-    case 0: hipLaunchKernelGGL((decode_mfma_kernel<T, G, kDecPref, kDecWaves, 0>), grid, block, 0, stream, p); break;
-    case kFogBias: hipLaunchKernelGGL((decode_mfma_kernel<T, G, kDecPref, kDecWaves, kFogBias>), grid, block, 0, stream, p); break;
-    case kFogVs: hipLaunchKernelGGL((decode_mfma_kernel<T, G, kDecPref, kDecWaves, kFogVs>), grid, block, 0, stream, p); break;
-    default:
-      hipLaunchKernelGGL((decode_mfma_kernel<T, G, kDecPref, kDecWaves, kFogBias | kFogVs>), grid, block, 0, stream, p);
+  switch ((p.bias ? kFogBias : 0) | (p.vscale ? kFogVs : 0)) {
+    case 0: launch_decode_one<T, GT, 0, D, kExact>(p, stream); break;
+    case kFogBias: launch_decode_one<T, GT, kFogBias, D, kExact>(p, stream); break;
+    case kFogVs: launch_decode_one<T, GT, kFogVs, D, kExact>(p, stream); break;
+    default: launch_decode_one<T, GT, kFogBias | kFogVs, D, kExact>(p, stream);
   }
   if (check_launch("fog decode (mfma)") != KESSIE_OK) return KESSIE_ERR_HIP;
   if (!p.direct_out && p.launch_combine) {
@@ -1670,9 +1717,10 @@ bool decode_mfma_ok(const Params& p, int dtype) {
   if (env_int("KESSIE_FORCE_GENERIC", 0)) return false;
   if (dtype != KESSIE_DTYPE_BF16 && dtype != KESSIE_DTYPE_F16 && dtype != KESSIE_DTYPE_F32) return false;
   // Pages of 16 * 2^k tokens (vLLM's 16, 32, 64, ... token blocks).
-  if (p.D != 128 || p.page_size < 16 || (p.page_size & (p.page_size - 1)) != 0 || p.page_table == nullptr)
-    return false;
-  if (!(p.G == 1 || p.G == 2 || p.G == 4 || p.G == 8 || p.G == 16)) return false;
+  if (p.page_size < 16 || (p.page_size & (p.page_size - 1)) != 0 || p.page_table == nullptr) return false;
+  if (p.G < 1 || p.G > 16) return false;
+  if (p.D != 128 && p.D != 64) return false;
+  if (dtype == KESSIE_DTYPE_F32 && (p.D != 128 || (p.G & (p.G - 1)) != 0)) return false;
   if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v) || !aligned16(p.out)) return false;
   // 16-byte rows: 8 elements of bf16/fp16, 4 of fp32.
   const int64_t vec = dtype == KESSIE_DTYPE_F32 ? 4 : 8;
@@ -1684,6 +1732,7 @@ bool decode_mfma_ok(const Params& p, int dtype) {
 
 template <typename T>
 int run_decode_mfma(Params& p, hipStream_t s) {
+  if (p.D == 64) return launch_decode_mfma<T, 0, 64, true>(p, s);
   switch (p.G) {
     case 1: return launch_decode_mfma<T, 1>(p, s);
     case 2: return launch_decode_mfma<T, 2>(p, s);
@@ -1691,8 +1740,7 @@ int run_decode_mfma(Params& p, hipStream_t s) {
     case 8: return launch_decode_mfma<T, 8>(p, s);
     case 16: return launch_decode_mfma<T, 16>(p, s);
   }
-  set_error(KESSIE_ERR_UNSUPPORTED, "fog decode: GQA ratio %d", p.G);
-  return KESSIE_ERR_UNSUPPORTED;
+  return launch_decode_mfma<T, 0, 128, true>(p, s);
 }
 
 int validate_common(const Params& p, int dtype) {

@@ -175,14 +175,7 @@ __device__ __forceinline__ float max_xor32(float x) {
 
 // max over the wave's lanes, in every lane (DPP within the rows of 16).
 __device__ __forceinline__ float wave_max(float x) {
-  auto dpp = [](float v, auto ctrl) {
-    return __builtin_bit_cast(
-        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  x = fmaxf(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // quad_perm 1,0,3,2
-  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // quad_perm 2,3,0,1
-  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
-  x = fmaxf(x, dpp(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+  x = row_max16(x);
   auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l)); };
   return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
 }

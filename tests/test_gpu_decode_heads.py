@@ -1,0 +1,80 @@
+"""GPU parity of decode on head_dim 64 and on GQA ratios that are no power of
+two: MFMA instances whose probabilities keep fp32 precision.
+
+Tolerance: the kernel's own error is that of fp32 sums (2e-5 of the result's
+norm), so the distance from the oracle is that of rounding the oracle's result
+to the type, and no more."""
+import pytest
+import torch
+
+from oracle.attention import paged_decode_ref
+from oracle.fog import fog_bias
+from tests.inputs import decode_case, gen, randn
+
+pytestmark = pytest.mark.gpu
+
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+def _check(out, q, pool, table, lens, vs, bias, window, dtype):
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        row = table[i].long()[: -(-n // pool.shape[1])].cpu()
+        ref = paged_decode_ref(q[i:i + 1].cpu(), pool[row.to(pool.device)].cpu(), torch.arange(len(row)).int()[None],
+                               torch.tensor([n]), None if vs is None else vs.view(-1, vs.shape[-1])[i % vs.shape[0]].cpu(),
+                               None if bias is None else bias[i:i + 1].cpu(), window)
+        err = (out[i:i + 1].double().cpu() - ref.double()).norm()
+        rounding = (ref.to(dtype).double() - ref.double()).norm()
+        assert err <= 1.05 * rounding + 2e-5 * ref.double().norm(), f"sequence {i} ({n} tokens): {err:.3e} {rounding:.3e}"
+
+
+@pytest.mark.parametrize("hq,hkv,d,ctx,lens,page,window,fog,dt", [
+    (32, 8, 64, 300, [300, 1, 15, 16, 17, 0, 64], 16, 0, "vscale", "bf16"),
+    (3, 3, 64, 700, [700, 31], 32, 0, "none", "fp16"),             # an odd number of kv heads, larger pages
+    (16, 1, 64, 5000, [5000], 16, 100, "bias", "bf16"),            # GQA 16, window, one sequence
+    (14, 2, 64, 400, [400, 399], 64, 33, "both", "fp16"),          # GQA 7
+    (24, 8, 128, 900, [900, 77, 16], 16, 0, "both", "bf16"),       # GQA 3
+    (12, 1, 128, 2000, [2000, 5], 32, 500, "vscale", "fp16"),      # GQA 12
+    (32, 8, 64, 9000, [9000] + [40 + 9 * i for i in range(30)], 16, 0, "bias", "bf16"),   # balanced splits
+    (24, 8, 128, 9000, [9000] + [40 + 9 * i for i in range(15)], 16, 0, "vscale", "fp16"),
+])
+def test_decode_exact_p_shapes(dev, hq, hkv, d, ctx, lens, page, window, fog, dt):
+    from kessie_amd import ops
+
+    b, dtype = len(lens), DT[dt]
+    q, pool, table, lens_d = decode_case(b, hq, hkv, d, ctx, page, dtype, dev, seed=51, ctx_lens=lens)
+    vs = torch.rand(b, ctx, generator=gen(dev, 52), device=dev) if fog in ("vscale", "both") else None
+    bias = fog_bias(ctx, 0.5, 0.5, {3, 17}, 0.1).to(dev).repeat(b, 1) if fog in ("bias", "both") else None
+    out = torch.full_like(q, float("nan"))
+    ops.fog_decode(q, pool, table, lens_d, ctx, fog_vscale=vs, fog_bias=bias, window=window, out=out)
+    torch.cuda.synchronize()
+    _check(out, q, pool, table, lens, vs, bias, window, dtype)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (6, 2, 128)])
+@pytest.mark.parametrize("lo,hi,vmul", [(1e4, 1e4, 1.0), (1e-6, 1e-6, 1e3), (1e-6, 1e4, 1.0), (-900.0, 900.0, 1.0)])
+def test_decode_fp16_weights_of_any_magnitude(dev, hq, hkv, d, lo, hi, vmul):
+    """V weights far from 1 (constant, or rising or changing sign along the context): p * w leaves fp16's range."""
+    from kessie_amd import ops
+
+    lens = [500, 33]
+    q, pool, table, lens_d = decode_case(2, hq, hkv, d, 500, 16, torch.float16, dev, seed=53, ctx_lens=lens)
+    pool, q = pool * vmul, q / vmul
+    ramp = torch.linspace(0, 1, 500, device=dev)
+    w = (lo + (hi - lo) * ramp if lo * hi < 0 else lo * (hi / lo) ** ramp).float().view(1, -1)
+    out = ops.fog_decode(q, pool, table, lens_d, 500, fog_vscale=w.view(-1))
+    _check(out, q, pool, table, lens, w, None, 0, torch.float16)
+
+
+def test_decode_exact_p_invalid_page(dev):
+    from kessie_amd import ops
+
+    q, pool, table, lens = decode_case(2, 12, 4, 64, 200, 16, torch.bfloat16, dev, seed=54, ctx_lens=[200, 100])
+    bad = table.clone()
+    bad[0, 3], bad[1, 0] = -1, pool.shape[0]
+    out = ops.fog_decode(q, pool, bad, lens, 200)
+    hide = torch.zeros(2, 200, device=dev)  # their tokens contribute nothing
+    hide[0, 48:64], hide[1, :16] = -float("inf"), -float("inf")
+    _check(out, q, pool, table, [200, 100], None, hide, 0, torch.bfloat16)
