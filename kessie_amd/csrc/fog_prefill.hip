@@ -537,7 +537,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   // The bias enters the scores as the products' starting value, in their units
   // (bias / sm_scale): one multiply-add per score less, and no pass over the
   // scores before their maximum (2,048 bf16 queries on 32,768 tokens at
-  // head_dim 128 1,043 -> 1,024 us, at 64 992 -> 940).  Not with
+  // head_dim 128 1,034 -> 1,026 us, at 64 985 -> 959).  Not with
   // kExactP at head_dim 128, which has no registers left (1,836 -> 1,943).
   constexpr bool kBiasC = kBias && !(kExactP && kD == 128);
   const float inv_scale = kBiasC ? 1.0f / p.sm_scale : 0.0f;
@@ -622,6 +622,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   float m_run = kNegInf, l_half = 0.0f;
   float e_run = -(float)kWRange;  // (kWExp)
   const float c2 = p.sm_scale * kLog2e;
+  const float slack = kBiasC ? fminf(kRescaleSlack / c2, 1e30f) : kRescaleSlack;
 
   // Tiles whose 64 keys all lie in [lo, hi) and are visible to every row of
   // the workgroup (causal: none after the first row's position; window: none
@@ -701,13 +702,25 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         mb = max3(mb, sc(kb)[v + 2], sc(kb)[v + 3]);
       }
     float mloc = max_xor32(fmaxf(ma, mb));
-    if (!kBiasY) mloc *= c2;  // c2 > 0
+    // (kBiasC: the running max stays in the units of x.)
+    if (!kBias) mloc *= c2;  // c2 > 0
     // The reference max moves only when a row's max rises by more than
     // kRescaleSlack (log2 units); until then p = 2^(y - m_run) <= 2^kRescaleSlack,
     // as exact in T as any p <= 1, and the O accumulators are left alone.
-    const float mnew = mloc > m_run + kRescaleSlack ? mloc : m_run;
-    float muse = mnew == kNegInf ? 0.0f : mnew;
-    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
+    const float mnew = mloc > m_run + slack ? mloc : m_run;
+    float muse = mnew == kNegInf ? 0.0f : kBiasC ? mnew * c2 : mnew;
+    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(kBiasC ? (m_run - mnew) * c2 : m_run - mnew);
+    if constexpr (kBiasC) {
+      // A max so large (every key seen so far under a mask of -1e9 or lower)
+      // that the rounding of mnew * c2 would show: subtract it from the scores.
+      const bool far = fabsf(muse) > 1048576.0f;
+      if (__builtin_amdgcn_ballot_w64(far) != 0) {
+        const float off = far ? mnew : 0.0f;
+        c0 -= off;
+        c1 -= off;
+        if (far) muse = 0.0f;
+      }
+    }
     if constexpr (kWExp) {
       const int we = ((int)(__builtin_bit_cast(uint32_t, fwm[st_cur]) >> 23) & 255) - 127;  // floor(log2), uniform
       const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
@@ -844,7 +857,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         *reinterpret_cast<f32x4*>(dst + 32 * db + 8 * vq) =
             f32x4{oacc[db][4 * vq], oacc[db][4 * vq + 1], oacc[db][4 * vq + 2], oacc[db][4 * vq + 3]};
     if (half == 0) {
-      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m_run + e_run : m_run) * kLn2;
+      const float m2 = kBiasC ? m_run * c2 : m_run;
+      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m2 + e_run : m2) * kLn2;
       p.ws_l[r] = l;
     }
     return;

@@ -100,17 +100,19 @@ def test_prefill_fp16_weights_of_any_magnitude(dev, monkeypatch, hq, hkv, d, spl
 
 
 @pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (8, 2, 128), (6, 2, 128)])
-@pytest.mark.parametrize("low", [-1e38, -65504.0, -float("inf")])
-def test_prefill_bias_masks(dev, hq, hkv, d, low):
+@pytest.mark.parametrize("low", [-1e38, -1e9, -65504.0, -float("inf")])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_prefill_bias_masks(dev, monkeypatch, hq, hkv, d, low, splits):
     """Keys hidden by the lowest values a mask holds (the bias enters the scores divided by sm_scale), and with
     the finite ones a sequence whose keys are all hidden alike."""
     from kessie_amd import ops
 
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
     _, pool, table, lens = decode_case(2, hq, hkv, d, 300, 16, torch.bfloat16, dev, seed=19, ctx_lens=[300, 300])
     q = randn((2, 70, hq, d), torch.bfloat16, dev, 20)
     bias = fog_bias(300, 0.5, 0.5, {3}, 0.1).to(dev).repeat(2, 1)
     bias[0, 5:100] = low
-    if low == -1e38:
+    if low in (-1e38, -1e9):  # (fp32 spacing there is above any score: all keys alike)
         bias[1] = low
     out = ops.fog_prefill(q, pool, table, lens, 300, fog_bias=bias)
     ref = paged_prefill_ref(q.cpu(), pool.cpu(), table.cpu(), lens.cpu(), None, bias.cpu(), 0)
