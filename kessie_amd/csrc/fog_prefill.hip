@@ -288,7 +288,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       if (qtile < before + total) {
         const int l = __ffsll((unsigned long long)__ballot(before + inc > qtile)) - 1;
         found = b0 + l;
-        qtile -= before + __builtin_amdgcn_readlane(inc - nt, l);
+        // Each sequence's last (longest) query tile first, so that the grid ends
+        // on short ones (two-layer steps with four prompts of 277-1,111: head_dim
+        // 64 242 -> 224 us, 128 241 -> 224; five fresh ones of up to 2,048, 289
+        // both ways).
+        qtile = before + __builtin_amdgcn_readlane(inc, l) - 1 - qtile;
         break;
       }
       before += total;
