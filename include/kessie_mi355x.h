@@ -146,6 +146,20 @@ int kessie_fog_decode_paged(
     int page_size, int max_ctx, int window, float sm_scale, int dtype,
     void* workspace, size_t workspace_bytes, void* stream);
 
+/* kessie_fog_decode_paged for a batch whose lengths the host knows: seen_total
+ * is the sum over the sequences of min(ctx_lens[b], window or ctx_lens[b])
+ * (0: not known).  It chooses how the batch is split over the device, not
+ * what is computed: any value gives a correct result. */
+int kessie_fog_decode_batch(
+    const void* q, const void* kv_pool, int num_pages, int64_t page_stride,
+    int64_t tok_stride,
+    int64_t kv_stride, int64_t head_stride, const int32_t* page_table,
+    int64_t table_stride, const int32_t* ctx_lens, const float* fog_vscale,
+    int64_t fog_vscale_bstride, const float* fog_bias, int64_t fog_bias_bstride,
+    void* out, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+    int page_size, int max_ctx, int window, float sm_scale, int dtype,
+    int64_t seen_total, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Size of the static device scratch of kessie_fog_decode_paged_noalloc. */
 #define KESSIE_DECODE_NOALLOC_SCRATCH_BYTES (16u << 20)
 

@@ -477,16 +477,19 @@ inline int combine_dsplit(int64_t rows, int D) {
   return y;
 }
 
-// combine_kernel with every load issued first (S <= 256 splits, at most
-// kAheadLoads per thread, plain split layout): lane s of wave 0 holds (m, l)
-// of splits s, s + 64, ..., and each thread the float2 column of its split
-// group, all requested before the first use, where combine_kernel waits for
-// the maxima, then for (m, l) again, then for the partials (three round trips
-// instead of one; a 4K-token decode's combine is latency-bound).  The same
-// arithmetic in the same order as combine_kernel's fast path -- max and sum
-// over lanes s, s + 64, ... then the same butterfly, each group's splits
-// summed in increasing order, the groups met by the same sum_groups -- so the
-// two give the same bits.
+// combine_kernel with every load issued first (up to 256 splits): lane s of
+// wave 0 holds (m, l) of splits s, s + 64, ..., and each thread the float2
+// column of its split group's first kAheadLoads splits, all requested before
+// the first use, where combine_kernel waits for the maxima, then for (m, l)
+// again, then for the partials (three round trips instead of one; a 4K-token
+// decode's combine is latency-bound).  A balanced row's place among the units
+// is found by every wave for itself, without a barrier, and its splits past
+// the first kAheadLoads of a group are read in a loop (12 sequences of 3,000
+// in a balanced step: 34.3 -> 33.8 us).
+// The same arithmetic in the same order as combine_kernel's fast path -- max
+// and sum over lanes s, s + 64, ... then the same butterfly, each group's
+// splits summed in increasing order, the groups met by the same sum_groups --
+// so the two give the same bits.
 constexpr int kAheadLoads = 8;
 
 template <typename T, bool TREE>
@@ -495,7 +498,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
   __shared__ float2 part[kCombineThreads];
   __shared__ float inv_l;
   const int64_t row = blockIdx.x;  // (b*C + i)*Hq + h
-  const int S = p.num_splits;
+  int S = p.num_splits;
   const int D = p.D;
   const int h = (int)(row % p.Hq);
   const int64_t bi = row / p.Hq;
@@ -509,7 +512,14 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
   }
   i += p.q0_off;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t first = row * S;
+  int64_t first = row * S;
+  if (p.balanced) {
+    const BatchPages bp = batch_pages(p);
+    const int P = decode_unit_pages(bp, p.units, p.B);
+    int u0;
+    decode_units_of_seq(bp, P, __builtin_amdgcn_readfirstlane(b), &u0, &S);
+    first = (int64_t)h * p.units + u0;
+  }
   const int chunk = D / gridDim.y;
   const int d0 = blockIdx.y * chunk;
   const int cols = chunk / 2, groups = kCombineThreads / cols;
@@ -561,6 +571,12 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
       ay += e * v[j].y;
     }
   }
+  for (int sp = grp + kAheadLoads * groups; sp < S; sp += groups) {  // (balanced rows only)
+    const float e = e_s[sp];
+    const float2 w = *reinterpret_cast<const float2*>(o + (int64_t)sp * D);
+    ax += e * w.x;
+    ay += e * w.y;
+  }
   const float2 acc = sum_groups<TREE>(ax, ay, tid, cols, groups, part);
   if (tid < cols) {
     store_out<T>(p, b, i, h, d0 + 2 * tid, acc.x * il);
@@ -569,8 +585,8 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
 }
 
 // The per-row merge of split partials: combine_ahead_kernel where its loads
-// fit (plain split layout, S <= 256, an even chunk dividing the workgroup,
-// S <= groups * kAheadLoads), else combine_kernel.  Same bits either way.
+// fit (an even chunk dividing the workgroup; up to 256 splits, balanced or at
+// most groups * kAheadLoads), else combine_kernel.  Same bits either way.
 // Decode sums the split groups as a tree; the prefill combines (TREE false)
 // in split order, which keeps varlen and per-sequence launches bit-equal.
 template <typename T, bool TREE = true>
@@ -578,8 +594,8 @@ void launch_row_combine(const Params& p, int64_t rows, hipStream_t s) {
   const int y = combine_dsplit(rows, p.D);
   const int chunk = p.D / y;
   const int S = p.num_splits;
-  bool ahead = !p.balanced && S <= 256 && (chunk & 1) == 0 && kCombineThreads % (chunk / 2) == 0;
-  if (ahead) ahead = S <= (kCombineThreads / (chunk / 2)) * kAheadLoads;
+  bool ahead = (p.balanced ? p.units : S) <= 256 && (chunk & 1) == 0 && kCombineThreads % (chunk / 2) == 0;
+  if (ahead && !p.balanced) ahead = S <= (kCombineThreads / (chunk / 2)) * kAheadLoads;
   if (ahead)
     hipLaunchKernelGGL((combine_ahead_kernel<T, TREE>), dim3((unsigned)rows, y), dim3(kCombineThreads), 0, s, p);
   else
@@ -1779,13 +1795,16 @@ namespace kessie {
 namespace attn {
 
 // Shared body of the decode entry points.  partials_only: write (m, l, o) per
-// split into the workspace and skip the combine.
+// split into the workspace and skip the combine.  seen_total: the tokens that the
+// batch sees in all where the caller knows them (0: not known); it chooses the
+// splits and nothing else.
 static int decode_entry(const void* q, const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,
                         int64_t kv_stride, int64_t head_stride, const int32_t* page_table, int64_t table_stride,
                         const int32_t* ctx_lens, const float* fog_vscale, int64_t fog_vscale_bstride,
                         const float* fog_bias, int64_t fog_bias_bstride, void* out, int batch, int num_q_heads,
                         int num_kv_heads, int head_dim, int page_size, int max_ctx, int window, float sm_scale,
-                        int dtype, void* workspace, size_t workspace_bytes, void* stream, bool partials_only) {
+                        int dtype, void* workspace, size_t workspace_bytes, void* stream, bool partials_only,
+                        int64_t seen_total = 0) {
   clear_error();
   Params p{};
   const int es = dtype_size(dtype);
@@ -1852,11 +1871,17 @@ static int decode_entry(const void* q, const void* kv_pool, int num_pages, int64
     // set-up costs each wave ~1 us before the first page load, so it is taken
     // for batches of 2..kBalSeqs sequences whose bound on the K/V bytes (B
     // times max_ctx tokens, or the window's) streams for at least ~40 us, 256
-    // MiB; one sequence, or a batch that small, gets the plain split.
+    // MiB, or lies 24 MiB or more above the bytes that are really read: 12
+    // sequences of 600-6,000 at head_dim 64 33.5 -> 23.0 us, of 300-3,000 at
+    // 128 27.1 -> 23.4, 24 of 100-1,000 21.0 -> 18.2 (equal lengths of those
+    // sizes would lose 1.2 us).  One sequence, or a batch that small, gets the
+    // plain split.
     const int seen = window > 0 ? min(window, max_ctx) : max_ctx;
-    const double kv_bound = (double)batch * seen * num_kv_heads * head_dim * 2.0 * dtype_size(dtype);
+    const double kv_token = num_kv_heads * head_dim * 2.0 * dtype_size(dtype);
+    const double kv_bound = (double)batch * seen * kv_token;
+    const double kv_spare = seen_total > 0 ? kv_bound - (double)seen_total * kv_token : 0.0;
     p.balanced = (!partials_only && !p.direct_out && batch >= 2 && batch <= kBalSeqs &&
-                  kv_bound >= 256.0 * 1024 * 1024) ? 1 : 0;
+                  (kv_bound >= 256.0 * 1024 * 1024 || kv_spare >= 24.0 * 1024 * 1024)) ? 1 : 0;
     p.units = p.balanced ? decode_units(batch, num_kv_heads, target, bound) : 0;
     if (dtype == KESSIE_DTYPE_F32) return run_decode_mfma_f32(p, s);
     return dtype == KESSIE_DTYPE_BF16 ? run_decode_mfma<bf16_t>(p, s) : run_decode_mfma<f16_t>(p, s);
@@ -1879,6 +1904,21 @@ extern "C" int kessie_fog_decode_paged(const void* q, const void* kv_pool, int n
                                     page_table, table_stride, ctx_lens, fog_vscale, fog_vscale_bstride, fog_bias,
                                     fog_bias_bstride, out, batch, num_q_heads, num_kv_heads, head_dim, page_size,
                                     max_ctx, window, sm_scale, dtype, workspace, workspace_bytes, stream, false);
+}
+
+extern "C" int kessie_fog_decode_batch(const void* q, const void* kv_pool, int num_pages, int64_t page_stride,
+                                       int64_t tok_stride, int64_t kv_stride, int64_t head_stride,
+                                       const int32_t* page_table, int64_t table_stride, const int32_t* ctx_lens,
+                                       const float* fog_vscale, int64_t fog_vscale_bstride, const float* fog_bias,
+                                       int64_t fog_bias_bstride, void* out, int batch, int num_q_heads,
+                                       int num_kv_heads, int head_dim, int page_size, int max_ctx, int window,
+                                       float sm_scale, int dtype, int64_t seen_total, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+  return kessie::attn::decode_entry(q, kv_pool, num_pages, page_stride, tok_stride, kv_stride, head_stride,
+                                    page_table, table_stride, ctx_lens, fog_vscale, fog_vscale_bstride, fog_bias,
+                                    fog_bias_bstride, out, batch, num_q_heads, num_kv_heads, head_dim, page_size,
+                                    max_ctx, window, sm_scale, dtype, workspace, workspace_bytes, stream, false,
+                                    seen_total);
 }
 
 extern "C" int kessie_fog_decode_partials(const void* q, const void* kv_pool, int num_pages, int64_t page_stride,

@@ -501,8 +501,8 @@ class KeSSieAttentionImpl:
         # Fog bias per sequence (row b built for that sequence's own length),
         # rows read with a batch stride by the kernels.
         bias = None
+        lens_host = getattr(meta, "seq_lens_cpu", None)
         if state is not None and kv_len > 0 and nseq > 0:
-            lens_host = getattr(meta, "seq_lens_cpu", None)
             bias = _FOG_CACHE.get_fog_bias_rows(lens, kv_len, query.device, query.dtype, state,
                                                 lens_host[:nseq] if lens_host is not None else None)
 
@@ -510,10 +510,14 @@ class KeSSieAttentionImpl:
             if decode == list(range(decode[0], decode[0] + len(decode))):
                 lo, hi = decode[0], decode[-1] + 1
                 q_dec = q[qsl[lo]:qsl[lo] + (hi - lo)]
+                seen = 0  # tokens the decode rows see, where the host knows them
+                if lens_host is not None and hi - lo > 1:
+                    w = self.window or kv_len
+                    seen = sum(min(n, w) for n in lens_host[lo:hi].tolist())
                 ops.fog_decode(q_dec, kv_cache, table[lo:hi], lens[lo:hi], kv_len,
                                fog_bias=None if bias is None else bias[lo:hi],
                                window=self.window, sm_scale=self.scale, layout=layout,
-                               out=out[qsl[lo]:qsl[lo] + (hi - lo)], stream=sp)
+                               out=out[qsl[lo]:qsl[lo] + (hi - lo)], stream=sp, seen_total=seen)
             else:
                 idx = torch.tensor(decode, device=q.device)
                 rows = torch.tensor([qsl[i] for i in decode], device=q.device)

@@ -168,11 +168,13 @@ def fog_decode(q: torch.Tensor, pool: torch.Tensor, page_table: torch.Tensor, ct
                fog_bias: Optional[torch.Tensor] = None, window: int = 0,
                sm_scale: Optional[float] = None, layout: str = "native",
                out: Optional[torch.Tensor] = None, ws: Optional[torch.Tensor] = None,
-               stream=None) -> torch.Tensor:
+               stream=None, seen_total: int = 0) -> torch.Tensor:
     """Fog decode: q [B, Hq, D] -> out [B, Hq, D] (q's dtype) over a paged pool.
 
     page_table int32 [B, W]; ctx_lens int32 [B] on the device; ``max_ctx`` is
-    a host-side upper bound of ctx_lens (it sizes the split-K grid).
+    a host-side upper bound of ctx_lens (it sizes the split-K grid);
+    ``seen_total``, where the host knows it, the sum of min(ctx_lens, window)
+    (it helps choose the splits of a batch of mixed lengths).
     """
     pv = pool_view(pool, layout)
     q = _contig(q, "q")
@@ -198,11 +200,11 @@ def fog_decode(q: torch.Tensor, pool: torch.Tensor, page_table: torch.Tensor, ct
     if ws is None:
         ws = workspace(need, q.device, "attn")
     wsz = 0 if ws is None else ws.numel() * ws.element_size()
-    _lib.check("kessie_fog_decode_paged", lib.kessie_fog_decode_paged(
+    _lib.check("kessie_fog_decode_batch", lib.kessie_fog_decode_batch(
         _ptr(q), C.c_void_p(pv.k_ptr), pv.num_pages, pv.page_stride, pv.tok_stride, pv.kv_stride,
         pv.head_stride, _ptr(page_table), page_table.stride(0), _ptr(ctx_lens), _ptr(vs), vs_bs,
         _ptr(bi), bi_bs, _ptr(out), b, hq, pv.num_kv_heads, d, pv.page_size, int(max_ctx), int(window),
-        float(sm_scale), dt, _ptr(ws), wsz, _stream_ptr(stream, q.device)))
+        float(sm_scale), dt, int(seen_total), _ptr(ws), wsz, _stream_ptr(stream, q.device)))
     return out
 
 

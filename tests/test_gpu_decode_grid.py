@@ -37,3 +37,29 @@ def test_decode_one_round_grid(dev, b, hkv, ctx, lens, window):
                                torch.tensor([n]), vs.cpu(), None, window)
         diff = (out[i:i + 1].float().cpu() - ref).abs()
         assert bool((diff <= 2e-2 + 1e-2 * ref.abs()).all()), f"sequence {i} ({n} tokens): {diff.max().item():.3e}"
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,dt,ctx,window", [
+    (12, 32, 8, 128, torch.bfloat16, 3000, 0), (12, 32, 8, 64, torch.float16, 6000, 0),
+    (24, 8, 2, 128, torch.float32, 4000, 0), (24, 24, 8, 128, torch.bfloat16, 2000, 1000),
+    (20, 32, 2, 128, torch.bfloat16, 9000, 0),  # 1,024 units a group of heads: the combine that loops
+])
+@pytest.mark.parametrize("total", ["sum", "one", "over"])
+def test_decode_known_lengths(dev, b, hq, hkv, d, dt, ctx, window, total):
+    """A total of the lengths given by the host chooses the balanced split below its size bound; any total
+    (here also 1, and more than the batch holds) leaves the result that of the plain split."""
+    from kessie_amd import ops
+
+    lens = [ctx] + [1 + (37 * i * i) % (ctx // 3) for i in range(1, b)]
+    q, pool, table, lens_d = decode_case(b, hq, hkv, d, ctx, 16, dt, dev, seed=43, ctx_lens=lens)
+    seen = {"sum": sum(min(n, window or n) for n in lens), "one": 1, "over": 2 * b * ctx}[total]
+    plain = ops.fog_decode(q, pool, table, lens_d, ctx, window=window)
+    out = ops.fog_decode(q, pool, table, lens_d, ctx, window=window, seen_total=seen)
+    diff = (out.float() - plain.float()).abs()
+    if dt != torch.float32 and d == 128 and hq // hkv in (4, 16):
+        # Probabilities rounded to the type against another running maximum (2^-9 each): this file's tolerance.
+        assert bool((diff <= 2e-2 + 1e-2 * plain.float().abs()).all()), diff.max().item()
+    else:
+        # One rounding of the output apart: only the splits' fp32 sums meet in another order.
+        tol = {torch.bfloat16: 2 ** -7, torch.float16: 2 ** -10, torch.float32: 2e-5}[dt]
+        assert bool((diff <= tol * (plain.float().abs() + 0.02)).all()), diff.max().item()
