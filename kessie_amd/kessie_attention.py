@@ -501,8 +501,9 @@ class KeSSieAttentionImpl:
         # Fog bias per sequence (row b built for that sequence's own length),
         # rows read with a batch stride by the kernels.
         bias = None
-        lens_host = getattr(meta, "seq_lens_cpu", None)
+        lens_host = None
         if state is not None and kv_len > 0 and nseq > 0:
+            lens_host = getattr(meta, "seq_lens_cpu", None)
             bias = _FOG_CACHE.get_fog_bias_rows(lens, kv_len, query.device, query.dtype, state,
                                                 lens_host[:nseq] if lens_host is not None else None)
 
