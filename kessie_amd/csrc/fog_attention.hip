@@ -18,8 +18,8 @@
 //                 one (sequence, split) x 2 kv heads, one wave per kv head; a
 //                 wave streams its kv head's K and V rows of every
 //                 page in its split with 16-byte loads (register prefetch of
-//                 PREF pages); QK^T and PV both on MFMA (P in the input
-//                 dtype, or as two operands of it, accumulation in fp32), V transposed through LDS.
+//                 PREF pages); QK^T and PV both on MFMA (P in the input dtype,
+//                 or to fp32 precision; accumulation in fp32), V transposed through LDS.
 //   attn_generic  any dtype / head_dim <= 256 / page size / GQA ratio: K and
 //                 V tiles staged in LDS as fp32, one workgroup per
 //                 (row tile, kv head, sequence, split).  Serves the shapes the
@@ -805,23 +805,73 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// x as three bf16 terms, h + m + l = x to 2^-23: h and m the upper halves of
+// the floats returned, l to be rounded.  They have x's sign and none is zero
+// where x is not, so that an infinite factor gives an infinity and not 0 * inf;
+// an infinite x is infinite in each.
+struct Bf16x3 {
+  uint32_t h, m;
+  float l;
+};
+template <bool kFinite>
+__device__ __forceinline__ Bf16x3 split_bf16(float x) {
+  constexpr float kTiny = 0x1p-26f;
+  const bool inf = !kFinite && fabsf(x) > 3.402823466e38f;
+  const uint32_t h = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
+  const float r = inf ? x : fmaf(x, kTiny, x - __builtin_bit_cast(float, h));
+  const uint32_t m = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+  return {h, m, inf ? x : fmaf(x, kTiny, r - __builtin_bit_cast(float, m))};
+}
+// The upper halves of two words, packed.
+__device__ __forceinline__ uint32_t upper2(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302); }
+
 // FOG: which per-token fog vectors the instance reads (bit 0 the logit bias,
 // bit 1 the V-scale); each one read costs a register per prefetched page.
 constexpr int kFogBias = 1, kFogVs = 2;
 
-// GT 0: any GQA ratio up to 16 (p.G).  kExact: p * w enters PV as two operands
-// of T, the rounded value and what the rounding left (p to 2^-16 relative in
-// bf16, 2^-22 in fp16), for the shapes the fp32 VALU kernel served before:
-// head_dim 64 and GQA ratios that are no power of two.  The loop waits on K
-// and V, not on the extra MFMAs.  Steps on the VALU kernel and here: head_dim
-// 64, 16 sequences of 131,072 tokens (32 q / 8 kv) 6,880 and 763 us (5.6 TB/s),
-// 12 of 600-6,000 143 and 36; head_dim 128 at GQA 3, 8 of 13,000-65,536
-// 2,454 and 174 (6.3 TB/s).
-// In fp16 with V weights, p * w is held in range by an exponent of the largest
-// weight so far, e_run, which scales O, the softmax sum and the stored max
-// alike; it moves when a page's weights exceed it by 2^kWSlack.
-constexpr int kWRange = 60;
-constexpr int kWSlack = 7;
+// GT 0: any GQA ratio up to 16 (p.G).  kExact: p * w enters PV to fp32
+// precision, for the shapes the fp32 VALU kernel served before: head_dim 64 and
+// GQA ratios that are no power of two.  bf16: as three bf16 terms, two of them
+// in one MFMA of twice the depth.  fp16, whose terms would share fp16's range
+// (a key 12 nats below the largest kept 8 bits): in fp32, V widened, on
+// v_mfma_f32_16x16x4_f32.  As on the VALU kernel, a key whose p is zero takes no
+// part whatever its weight, and infinities in V and the weights carry through.
+// The next loads go out before the products, which are longer here (head_dim
+// 64 782 -> 694 us at 16 x 131,072, fp16 450 -> 379 at 16 x 65,536).  Steps on
+// the VALU kernel and here: head_dim 64, 16 sequences of 131,072 tokens (32 q /
+// 8 kv, bf16) 6,880 and 694 us (6.2 TB/s), 12 of 600-6,000 143 and 32;
+// head_dim 128 at GQA 3, 8 of 13,000-65,536 2,454 and 174 (fp16 179).
+// x as three bf16 terms, h + m + l = x to 2^-23: h and m the upper halves of
+// the floats returned, l to be rounded.  They have x's sign and none is zero
+// where x is not, so that an infinite factor gives an infinity and not 0 * inf;
+// an infinite x is infinite in each.
+struct Bf16x3 {
+  uint32_t h, m;
+  float l;
+};
+template <bool kFinite>
+__device__ __forceinline__ Bf16x3 split_bf16(float x) {
+  constexpr float kTiny = 0x1p-26f;
+  const bool inf = !kFinite && fabsf(x) > 3.402823466e38f;
+  const uint32_t h = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
+  const float r = inf ? x : fmaf(x, kTiny, x - __builtin_bit_cast(float, h));
+  const uint32_t m = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+  return {h, m, inf ? x : fmaf(x, kTiny, r - __builtin_bit_cast(float, m))};
+}
+// The upper halves of two words, packed.
+__device__ __forceinline__ uint32_t upper2(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302); }
+
+// FOG: which per-token fog vectors the instance reads (bit 0 the logit bias,
+// bit 1 the V-scale); each one read costs a register per prefetched page.
+constexpr int kFogBias = 1, kFogVs = 2;
+
+// GT 0: any GQA ratio up to 16 (p.G).  kExact: p * w and V enter PV in fp32, on
+// v_mfma_f32_16x16x4_f32, as on the fp32 VALU kernel that serves the other
+// shapes (a key whose p is zero takes no part whatever its weight, infinities
+// in V and in the weights carry through): head_dim 64 and GQA ratios that are
+// no power of two.  Two 16-bit operands of p would share fp16's range, and a
+// key 12 nats below the largest kept 8 of its bits.  The loop waits on K and V,
+// not on the slower MFMAs.  Steps on the VALU kernel and here: @@
 
 template <typename T, int GT, int PREF, int W, int FOG, int D, bool kExact>
 // Two waves per SIMD (256 VGPRs; ~160 used with two pages of K and V in flight).
@@ -833,7 +883,6 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   constexpr int kCh = D / 8;     // 16-byte chunks of a row
   constexpr int kVL = D / 32;    // V loads per page, 64 / kCh tokens each
   constexpr int kBlk = D / 16;   // O^T blocks
-  constexpr bool kWExp = kExact && (FOG & kFogVs) != 0 && std::is_same<T, f16_t>::value;
   const int G = GT ? GT : p.G;
   __shared__ __align__(16) T vtile_all[W][16 * kVRow];
   __shared__ __align__(16) T qtile_all[W][16 * kVRow];
@@ -909,8 +958,6 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   for (int blk = 0; blk < kBlk; ++blk) oacc[blk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = kNegInf, l_run = 0.0f;  // softmax state of head `row`
 
-  float e_run = -(float)kWRange;          // (kWExp)
-
   vec8 kreg[PREF][kKB], vreg[PREF][kVL];
   int pid_s[PREF];
   // Per-token fog values of the next page to compute, lane t (< 16) holding
@@ -946,6 +993,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
   };
 
+  // What page lp's stage takes when it is done: the next page's fog values, then page lp + PREF.
+  auto next = [&](int st, int lp) {
+    if (FOG && lp + 1 < p1) load_fog(lp + 1);
+    if (lp + PREF < p1) issue(st, lp + PREF);
+  };
+
 #pragma unroll
   for (int st = 0; st < PREF; ++st)
     if (p0 + st < p1) issue(st, p0 + st);
@@ -958,8 +1011,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       if (lp >= p1) break;
       const int pid = pid_s[st];
       if (pid < 0 || pid >= p.num_pages) {  // masked page: contributes nothing
-        if (FOG && lp + 1 < p1) load_fog(lp + 1);
-        if (lp + PREF < p1) issue(st, lp + PREF);
+        next(st, lp);
         continue;
       }
       const int t_page = lp << 4;
@@ -984,22 +1036,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
       mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
       const float mnew = fmaxf(m_run, mloc);
-      float alpha = (m_run == kNegInf) ? 0.0f : __expf(m_run - mnew);
-      float wsc = 1.0f;  // 2^-e_run
-      if constexpr (kWExp) {
-        const float wm = row_max16(fabsf(fv_cur));  // lanes 0..15 hold the page's weights
-        const int we = ((int)(__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wm)) >> 23) & 255) - 127;
-        const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
-        alpha *= __builtin_amdgcn_exp2f(e_run - e_new);
-        wsc = __builtin_amdgcn_exp2f(-e_new);
-        e_run = e_new;
-      }
+      const float alpha = (m_run == kNegInf) ? 0.0f : __expf(m_run - mnew);
       float pr[4];
       float psum = 0.0f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         pr[i] = (sc[i] == kNegInf) ? 0.0f : __expf(sc[i] - mnew);
-        if constexpr (kWExp) pr[i] *= wsc;
         psum += pr[i];
       }
       psum += __shfl_xor(psum, 16);
@@ -1008,7 +1050,10 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       m_run = mnew;
       if (FOG & kFogVs) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pr[i] *= __shfl(fv_cur, 4 * grp + i);
+        for (int i = 0; i < 4; ++i) {
+          const float w = __shfl(fv_cur, 4 * grp + i);
+          pr[i] = kExact ? (pr[i] == 0.0f ? 0.0f : pr[i] * w) : pr[i] * w;
+        }
       }
       if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
@@ -1029,22 +1074,48 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
       for (int i = 0; i < kVL; ++i) *reinterpret_cast<vec8*>(vtile + vtok(i) * kVRow + 8 * vch) = vreg[st][i];
       wave_lds_sync();
-      vec4 pb, pl;
+      // (kExact: ahead of the longer products, so that the loads do not wait for them.)
+      if constexpr (kExact) next(st, lp);
+      if constexpr (kExact && std::is_same<T, bf16_t>::value) {
+        // p as three bf16 terms: two share an MFMA of twice the depth, V beside itself.
+        Bf16x3 t[4];
+        vec4 pl, va[kBlk];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pb[i] = static_cast<T>(pr[i]);
-        if constexpr (kExact) pl[i] = static_cast<T>(pr[i] - static_cast<float>(pb[i]));
+        for (int i = 0; i < 4; ++i) {
+          t[i] = split_bf16<(FOG & kFogVs) == 0>(pr[i]);
+          pl[i] = static_cast<T>(t[i].l);
+        }
+        const vec8 phm = __builtin_bit_cast(
+            vec8, (u32x4){upper2(t[0].h, t[1].h), upper2(t[2].h, t[3].h), upper2(t[0].m, t[1].m), upper2(t[2].m, t[3].m)});
+#pragma unroll
+        for (int blk = 0; blk < kBlk; ++blk) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) va[blk][i] = vtile[(4 * grp + i) * kVRow + 16 * blk + row];
+          oacc[blk] = Mfma<T>::mma32(__builtin_shufflevector(va[blk], va[blk], 0, 1, 2, 3, 4, 5, 6, 7), phm, oacc[blk]);
+        }
+#pragma unroll
+        for (int blk = 0; blk < kBlk; ++blk) oacc[blk] = Mfma<T>::mma16(va[blk], pl, oacc[blk]);
+      } else if constexpr (kExact) {
+        // MFMA i takes token 4 * grp + i of every lane group: V[token][d] and p[token][head].
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int blk = 0; blk < kBlk; ++blk)
+            oacc[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32(vtile[(4 * grp + i) * kVRow + 16 * blk + row]),
+                                                             pr[i], oacc[blk], 0, 0, 0);
+      } else {
+        vec4 pb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pb[i] = static_cast<T>(pr[i]);
+#pragma unroll
+        for (int blk = 0; blk < kBlk; ++blk) {
+          vec4 va;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) va[i] = vtile[(4 * grp + i) * kVRow + 16 * blk + row];
+          oacc[blk] = Mfma<T>::mma16(va, pb, oacc[blk]);
+        }
+        next(st, lp);
       }
-#pragma unroll
-      for (int blk = 0; blk < kBlk; ++blk) {
-        vec4 va;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) va[i] = vtile[(4 * grp + i) * kVRow + 16 * blk + row];
-        oacc[blk] = Mfma<T>::mma16(va, pb, oacc[blk]);
-        if constexpr (kExact) oacc[blk] = Mfma<T>::mma16(va, pl, oacc[blk]);
-      }
-      if (FOG && lp + 1 < p1) load_fog(lp + 1);
-      if (lp + PREF < p1) issue(st, lp + PREF);
     }
   }
 
@@ -1067,7 +1138,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
     for (int blk = 0; blk < kBlk; ++blk) *reinterpret_cast<f32x4*>(dst + 16 * blk) = oacc[blk];
     if (grp == 0) {
-      p.ws_m[slot] = kWExp ? m_run + e_run * 0.6931471805599453f : m_run;
+      p.ws_m[slot] = m_run;
       p.ws_l[slot] = l_run;
     }
   }

@@ -1,5 +1,5 @@
 """GPU parity of decode on head_dim 64 and on GQA ratios that are no power of
-two: MFMA instances whose probabilities keep fp32 precision.
+two: MFMA instances whose probabilities, weights and V enter PV in fp32.
 
 Tolerance: the kernel's own error is that of fp32 sums (2e-5 of the result's
 norm), so the distance from the oracle is that of rounding the oracle's result
@@ -9,7 +9,8 @@ import torch
 
 from oracle.attention import paged_decode_ref
 from oracle.fog import fog_bias
-from tests.inputs import decode_case, gen, randn
+from tests.exact64 import attend64, close_to_rounding, paged
+from tests.inputs import decode_case, gen
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +79,85 @@ def test_decode_exact_p_invalid_page(dev):
     hide = torch.zeros(2, 200, device=dev)  # their tokens contribute nothing
     hide[0, 48:64], hide[1, :16] = -float("inf"), -float("inf")
     _check(out, q, pool, table, [200, 100], None, hide, 0, torch.bfloat16)
+
+
+SHAPES = pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (6, 2, 128)])
+
+
+@SHAPES
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+def test_decode_small_probabilities(dev, monkeypatch, hq, hkv, d, dt):
+    """One key 12 above all others, with a small V (an attention sink): the result rests on probabilities of e^-12,
+    which 16-bit operands of fp16's range hold to a part in 1,000 only.  (One split: the sink is every key's.)"""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_DECODE_WGS", "1")
+    dtype, n = DT[dt], 4096
+    k = torch.zeros(n, hkv, d, device=dev, dtype=dtype)
+    k[5] = 12 / d ** 0.5
+    v = (1 + 0.1 * torch.randn(n, hkv, d, generator=gen(dev, 61), device=dev)).to(dtype)
+    v[5] = 2.0 ** -10
+    q = torch.ones(1, hq, d, device=dev, dtype=dtype)
+    pool, table, lens = paged(k, v)
+    close_to_rounding(ops.fog_decode(q, pool, table, lens, n), attend64(q, k, v, n - 1), dtype)
+
+
+@SHAPES
+@pytest.mark.parametrize("where", ["faint", "window"])
+def test_decode_fp16_one_large_weight(dev, hq, hkv, d, where):
+    """A weight of 2^16 on a key whose probability is negligible, or that the window hides, costs the others nothing."""
+    from kessie_amd import ops
+
+    n, window = 700, 500 if where == "window" else 0
+    k, v = (torch.randn(n, hkv, d, generator=gen(dev, 62 + i), device=dev).half() for i in (0, 1))
+    q = torch.randn(1, hq, d, generator=gen(dev, 64), device=dev).half()
+    w, bias = torch.ones(n, device=dev), torch.zeros(n, device=dev)
+    w[190] = 2.0 ** 16
+    if where == "faint":
+        bias[190] = -60.0
+    pool, table, lens = paged(k, v)
+    out = ops.fog_decode(q, pool, table, lens, n, fog_vscale=w, fog_bias=bias, window=window)
+    close_to_rounding(out, attend64(q, k, v, n - 1, w, bias, window), torch.float16)
+
+
+@SHAPES
+def test_decode_fp16_weights_under_a_mask(dev, hq, hkv, d):
+    """Every key under a mask of -1e9: the splits, whose weights differ, still count alike."""
+    from kessie_amd import ops
+
+    n = 1000
+    k = torch.zeros(n, hkv, d, device=dev, dtype=torch.float16)
+    v = torch.randn(n, hkv, d, generator=gen(dev, 65), device=dev).half()
+    q = torch.randn(1, hq, d, generator=gen(dev, 66), device=dev).half()
+    w = torch.logspace(0, -4, n, device=dev)
+    bias = torch.full((n,), -1e9, device=dev)
+    pool, table, lens = paged(k, v)
+    out = ops.fog_decode(q, pool, table, lens, n, fog_vscale=w, fog_bias=bias)
+    close_to_rounding(out, attend64(q, k, v, n - 1, w, bias), torch.float16)
+
+
+@SHAPES
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("what", ["v", "-v", "weight", "hidden weight"])
+def test_decode_infinities(dev, hq, hkv, d, dt, what):
+    """An infinity in V or in a weight shows as an infinity where its key takes part, and not at all where its
+    probability is zero."""
+    from kessie_amd import ops
+
+    dtype, n = DT[dt], 300
+    k, v = (torch.randn(n, hkv, d, generator=gen(dev, 67 + i), device=dev).to(dtype) for i in (0, 1))
+    q = torch.randn(1, hq, d, generator=gen(dev, 69), device=dev).to(dtype)
+    w, bias = torch.ones(n, device=dev), torch.zeros(n, device=dev)
+    if what.endswith("v"):
+        v[130, :, 3] = float("-inf" if what == "-v" else "inf")
+    else:
+        w[130] = float("inf")
+        if what == "hidden weight":
+            bias[130] = -float("inf")
+    pool, table, lens = paged(k, v)
+    out = ops.fog_decode(q, pool, table, lens, n, fog_vscale=w, fog_bias=bias).double().cpu()
+    ref = attend64(q, k, v, n - 1, w, bias)
+    finite = ref.isfinite()
+    assert finite.all() == (what == "hidden weight") and not ref.isnan().any()
+    assert torch.equal(out[~finite], ref[~finite])
+    close_to_rounding(torch.where(finite, out, 0.0), torch.where(finite, ref, 0.0), dtype)
