@@ -841,38 +841,6 @@ constexpr int kFogBias = 1, kFogVs = 2;
 // the VALU kernel and here: head_dim 64, 16 sequences of 131,072 tokens (32 q /
 // 8 kv, bf16) 6,880 and 694 us (6.2 TB/s), 12 of 600-6,000 143 and 32;
 // head_dim 128 at GQA 3, 8 of 13,000-65,536 2,454 and 174 (fp16 179).
-// x as three bf16 terms, h + m + l = x to 2^-23: h and m the upper halves of
-// the floats returned, l to be rounded.  They have x's sign and none is zero
-// where x is not, so that an infinite factor gives an infinity and not 0 * inf;
-// an infinite x is infinite in each.
-struct Bf16x3 {
-  uint32_t h, m;
-  float l;
-};
-template <bool kFinite>
-__device__ __forceinline__ Bf16x3 split_bf16(float x) {
-  constexpr float kTiny = 0x1p-26f;
-  const bool inf = !kFinite && fabsf(x) > 3.402823466e38f;
-  const uint32_t h = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
-  const float r = inf ? x : fmaf(x, kTiny, x - __builtin_bit_cast(float, h));
-  const uint32_t m = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
-  return {h, m, inf ? x : fmaf(x, kTiny, r - __builtin_bit_cast(float, m))};
-}
-// The upper halves of two words, packed.
-__device__ __forceinline__ uint32_t upper2(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302); }
-
-// FOG: which per-token fog vectors the instance reads (bit 0 the logit bias,
-// bit 1 the V-scale); each one read costs a register per prefetched page.
-constexpr int kFogBias = 1, kFogVs = 2;
-
-// GT 0: any GQA ratio up to 16 (p.G).  kExact: p * w and V enter PV in fp32, on
-// v_mfma_f32_16x16x4_f32, as on the fp32 VALU kernel that serves the other
-// shapes (a key whose p is zero takes no part whatever its weight, infinities
-// in V and in the weights carry through): head_dim 64 and GQA ratios that are
-// no power of two.  Two 16-bit operands of p would share fp16's range, and a
-// key 12 nats below the largest kept 8 of its bits.  The loop waits on K and V,
-// not on the slower MFMAs.  Steps on the VALU kernel and here: @@
-
 template <typename T, int GT, int PREF, int W, int FOG, int D, bool kExact>
 // Two waves per SIMD (256 VGPRs; ~160 used with two pages of K and V in flight).
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_mfma_kernel(Params p) {
