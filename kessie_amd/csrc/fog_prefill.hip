@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   extern __shared__ __align__(16) unsigned char smem[];
   T* ks = reinterpret_cast<T*>(smem);                                                // [stage][64][kKRow]
   uint32_t* vts = reinterpret_cast<uint32_t*>(smem + (size_t)kPfStages * kKStage * 2);  // [stage][128][kVRowW]
-  float* fbs = reinterpret_cast<float*>(vts + kPfStages * kVStage);                   // [stage][64] bias_in(bias)
+  float* fbs = reinterpret_cast<float*>(vts + kPfStages * kVStage);                   // [stage][64] bias*log2(e)
   float* fws = fbs + kPfStages * kPfKT;                                               // [stage][64] V weights (kExactP)
   float* fwm = fws + kPfStages * kPfKT;                                               // [stage] their max magnitude
   constexpr bool kWExp = kExactP && kVs && std::is_same<T, f16_t>::value;
@@ -538,19 +538,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   // probabilities stay unscaled and the softmax sum can be taken from them.
   // (kExactP: V stays as it is and the fp32 probabilities take the weights.)
   constexpr bool kScaleV = kVs && !kExactP;
-  // The bias enters the scores as the products' starting value, in their units
-  // (bias / sm_scale): one multiply-add per score less, and no pass over the
-  // scores before their maximum (2,048 bf16 queries on 32,768 tokens at
-  // head_dim 128 1,034 -> 1,026 us, at 64 985 -> 959).  Not with
-  // kExactP at head_dim 128, which has no registers left (1,836 -> 1,943).
-  constexpr bool kBiasC = kBias && !(kExactP && kD == 128);
-  const float inv_scale = kBiasC ? 1.0f / p.sm_scale : 0.0f;
-  // (A finite bias stays finite: masks of the type's lowest value.)
-  auto bias_in = [&](float b) {
-    if (!kBiasC) return b * kLog2e;
-    const float x = b * inv_scale;
-    return fabsf(b) < -kNegInf ? fmaxf(fminf(x, 3.402823466e38f), -3.402823466e38f) : x;
-  };
   auto store_weights = [&](int stage, int set) {
     if (kVs && kExactP && tid < kPfKT) {  // wave 0
       fws[stage * kPfKT + tid] = fk_r[set];
@@ -568,7 +555,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         vd[(8 * kc + e) * kVRowW] = kScaleV ? pack2<T>(to_f32(vreg[set][0][e]) * fw0[set], to_f32(vreg[set][1][e]) * fw1[set])
                                         : bits16(vreg[set][0][e]) | (bits16(vreg[set][1][e]) << 16);
     }
-    if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = bias_in(fb_r[set]);
+    if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
     store_weights(stage, set);
   };
 
@@ -585,24 +572,9 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       T* kd = ks + stage * kKStage + 8 * kc;
 #pragma unroll
       for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
-      if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = bias_in(fb_r[set]);
+      if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
       store_weights(stage, set);
     }
-  };
-  // What a tile's scores start from: zero, or the bias (kBiasC), read from LDS
-  // into the accumulators of the products.
-  auto score_init = [&](int stage, int kb) {
-    f32x16 r = {};
-    if constexpr (kBiasC) {
-      const float* fb = fbs + stage * kPfKT + 32 * kb + 8 * half;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(fb + 16 * (q >> 1) + 4 * (q & 1));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[4 * q + e] = x[e];
-      }
-    }
-    return r;
   };
   // S^T of the tile in a stage: lane (col, half) reads K row 32kb + col.
   const T* kread = ks + col * kKRow + 8 * half;
@@ -610,7 +582,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     const T* kb0 = kread + stage * kKStage;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      s[kb] = score_init(stage, kb);
+      s[kb] = f32x16{};
 #pragma unroll
       for (int st = 0; st < kDS; ++st)
         s[kb] = Mma32<T>::mma(*reinterpret_cast<const v8*>(kb0 + 32 * kb * kKRow + 16 * st), qv[st], s[kb]);
@@ -626,7 +598,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   float m_run = kNegInf, l_half = 0.0f;
   float e_run = -(float)kWRange;  // (kWExp)
   const float c2 = p.sm_scale * kLog2e;
-  const float slack = kBiasC ? fminf(kRescaleSlack / c2, 1e30f) : kRescaleSlack;
 
   // Tiles whose 64 keys all lie in [lo, hi) and are visible to every row of
   // the workgroup (causal: none after the first row's position; window: none
@@ -668,9 +639,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     ids_b = fetch_tile(t + 5);
 
     const bool interior = pm0 == 0xF && t >= ti_lo && t < ti_hi;
-    // Base-2 logits y = x * c2 (x holds the bias), or y itself (kBiasY); the tile max of y.
-    constexpr bool kBiasY = kBias && !kBiasC;
     const float* fbt = fbs + st_cur * kPfKT + 8 * half;
+    // Base-2 logits y = x * c2 (+ bias * log2 e); the tile max of y.
     if (!interior) {
       // This lane's keys of the tile form one interval of key offsets,
       // [klo_r, khi_r) relative to this lane's first key, intersected with
@@ -688,10 +658,10 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         for (int v = 0; v < 16; ++v) {
           const int kl = 32 * kb + 16 * (v >> 3) + (v & 7);  // key offset minus 8 * half
           const bool ok = ((uint32_t)(kl - off) < len) & (((pm0 >> (2 * kb + (v >> 3))) & 1) != 0);
-          const float y = kBiasY ? fmaf(sc(kb)[v], c2, fbt[32 * kb + 16 * (v >> 3) + (v & 7)]) : sc(kb)[v];
+          float y = kBias ? fmaf(sc(kb)[v], c2, fbt[32 * kb + 16 * (v >> 3) + (v & 7)]) : sc(kb)[v];
           sc(kb)[v] = ok ? y : kNegInf;
         }
-    } else if (kBiasY) {
+    } else if (kBias) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -706,25 +676,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         mb = max3(mb, sc(kb)[v + 2], sc(kb)[v + 3]);
       }
     float mloc = max_xor32(fmaxf(ma, mb));
-    // (kBiasC: the running max stays in the units of x.)
-    if (!kBias) mloc *= c2;  // c2 > 0
+    if (!kBias) mloc *= c2;  // without a bias, y = x * c2 and c2 > 0
     // The reference max moves only when a row's max rises by more than
     // kRescaleSlack (log2 units); until then p = 2^(y - m_run) <= 2^kRescaleSlack,
     // as exact in T as any p <= 1, and the O accumulators are left alone.
-    const float mnew = mloc > m_run + slack ? mloc : m_run;
-    float muse = mnew == kNegInf ? 0.0f : kBiasC ? mnew * c2 : mnew;
-    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(kBiasC ? (m_run - mnew) * c2 : m_run - mnew);
-    if constexpr (kBiasC) {
-      // A max so large (every key seen so far under a mask of -1e9 or lower)
-      // that the rounding of mnew * c2 would show: subtract it from the scores.
-      const bool far = fabsf(muse) > 1048576.0f;
-      if (__builtin_amdgcn_ballot_w64(far) != 0) {
-        const float off = far ? mnew : 0.0f;
-        c0 -= off;
-        c1 -= off;
-        if (far) muse = 0.0f;
-      }
-    }
+    const float mnew = mloc > m_run + kRescaleSlack ? mloc : m_run;
+    float muse = mnew == kNegInf ? 0.0f : mnew;
+    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
     if constexpr (kWExp) {
       const int we = ((int)(__builtin_bit_cast(uint32_t, fwm[st_cur]) >> 23) & 255) - 127;  // floor(log2), uniform
       const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
@@ -761,8 +719,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     auto exp_pair = [&](int j) {   // keys 2j, 2j+1 of this lane's 32
       const int kb = j >> 3, v = 2 * (j & 7);
       const float y0 = sc(kb)[v], y1 = sc(kb)[v + 1];
-      float p0 = __builtin_amdgcn_exp2f(kBiasY ? y0 - muse : fmaf(y0, c2, -muse));
-      float p1 = __builtin_amdgcn_exp2f(kBiasY ? y1 - muse : fmaf(y1, c2, -muse));
+      float p0 = __builtin_amdgcn_exp2f(kBias ? y0 - muse : fmaf(y0, c2, -muse));
+      float p1 = __builtin_amdgcn_exp2f(kBias ? y1 - muse : fmaf(y1, c2, -muse));
       if constexpr (kExactP) {
         ps0 += p0;
         ps1 += p1;
@@ -791,9 +749,9 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         // The next tile's second block into x, then its first into c0
         // (whose exponentials, the first eight pairs, are issued by then).
         if (i < kDS)
-          x = Mma32<T>::mma(op[i % 3], qv[i], i == 0 ? score_init(st_nxt, 1) : x);
+          x = Mma32<T>::mma(op[i % 3], qv[i], i == 0 ? f32x16{} : x);
         else
-          c0 = Mma32<T>::mma(op[i % 3], qv[i - kDS], i == kDS ? score_init(st_nxt, 0) : c0);
+          c0 = Mma32<T>::mma(op[i % 3], qv[i - kDS], i == kDS ? f32x16{} : c0);
       } else {
         const int s = (i - kQ) / kDB, db = (i - kQ) % kDB;
         oacc[db] = Mma32<T>::mma(op[i % 3], __builtin_bit_cast(v8, pb[s]), oacc[db]);
@@ -861,8 +819,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         *reinterpret_cast<f32x4*>(dst + 32 * db + 8 * vq) =
             f32x4{oacc[db][4 * vq], oacc[db][4 * vq + 1], oacc[db][4 * vq + 2], oacc[db][4 * vq + 3]};
     if (half == 0) {
-      const float m2 = kBiasC ? m_run * c2 : m_run;
-      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m2 + e_run : m2) * kLn2;
+      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m_run + e_run : m_run) * kLn2;
       p.ws_l[r] = l;
     }
     return;

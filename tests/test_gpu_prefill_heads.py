@@ -9,6 +9,7 @@ import torch
 
 from oracle.attention import paged_prefill_ref
 from oracle.fog import fog_bias
+from tests.exact64 import attend64, close_to_rounding, paged
 from tests.inputs import decode_case, gen, randn
 
 pytestmark = pytest.mark.gpu
@@ -103,8 +104,8 @@ def test_prefill_fp16_weights_of_any_magnitude(dev, monkeypatch, hq, hkv, d, spl
 @pytest.mark.parametrize("low", [-1e38, -1e9, -65504.0, -float("inf")])
 @pytest.mark.parametrize("splits", [1, 2])
 def test_prefill_bias_masks(dev, monkeypatch, hq, hkv, d, low, splits):
-    """Keys hidden by the lowest values a mask holds (the bias enters the scores divided by sm_scale), and with
-    the finite ones a sequence whose keys are all hidden alike."""
+    """Keys hidden by the lowest values a mask holds, and with the finite ones a sequence whose keys are all hidden
+    alike."""
     from kessie_amd import ops
 
     monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
@@ -118,3 +119,18 @@ def test_prefill_bias_masks(dev, monkeypatch, hq, hkv, d, low, splits):
     ref = paged_prefill_ref(q.cpu(), pool.cpu(), table.cpu(), lens.cpu(), None, bias.cpu(), 0)
     diff = (out.float().cpu() - ref).abs()
     assert bool((diff <= 2e-2 + 1e-2 * ref.abs()).all()), f"max diff {diff.max().item():.3e}"
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (8, 2, 128), (6, 2, 128)])
+def test_prefill_large_common_bias(dev, hq, hkv, d):
+    """A bias of -30,000 on every key leaves the softmax as it is but for one rounding of each logit, in base 2 to
+    2^-9 at most: p to ln 2 * 2^-9 = 1.4e-3, independently from key to key."""
+    from kessie_amd import ops
+
+    n, c = 600, 90
+    k, v = (torch.randn(n, hkv, d, generator=gen(dev, 31 + i), device=dev).half() for i in (0, 1))
+    q = torch.randn(1, c, hq, d, generator=gen(dev, 33), device=dev).half()
+    bias = torch.full((n,), -30000.0, device=dev)
+    pool, table, lens = paged(k, v)
+    out = ops.fog_prefill(q, pool, table, lens, n, fog_bias=bias)
+    close_to_rounding(out[0], attend64(q[0], k, v, n - c), torch.float16, own=1.4e-3)
