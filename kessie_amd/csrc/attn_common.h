@@ -95,18 +95,6 @@ __device__ __forceinline__ bool key_visible(int q_pos, int t, int window, int ca
   return true;
 }
 
-// max over the 16 lanes of a DPP row, in each of them.
-__device__ __forceinline__ float row_max16(float x) {
-#define KESSIE_DPP_MAX(ctrl) \
-  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xf, 0xf, false)))
-  KESSIE_DPP_MAX(0xB1);   // quad_perm 1,0,3,2
-  KESSIE_DPP_MAX(0x4E);   // quad_perm 2,3,0,1
-  KESSIE_DPP_MAX(0x141);  // row_half_mirror
-  KESSIE_DPP_MAX(0x140);  // row_mirror
-#undef KESSIE_DPP_MAX
-  return x;
-}
-
 // Row index into the partial workspace / output for (b, i, h).
 __device__ __forceinline__ int64_t row_id(const Params& p, int b, int i, int h) {
   return ((int64_t)b * p.C + i) * p.Hq + h;

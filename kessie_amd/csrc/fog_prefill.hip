@@ -35,17 +35,23 @@
 // sits on one XCD and the query tiles of that head share its keys in L2.
 //
 // Variants (template and Params):
-//   kExactP  the probabilities enter PV as two operands of T, the rounded value
-//            and what the rounding left (p to 2^-16 relative in bf16, 2^-22 in
-//            fp16), the V-fog weights multiply them in fp32 and V is not
-//            rescaled.  Twice the PV MFMAs, for the precision of the fp32 VALU
-//            kernel (attn_generic_kernel), which these shapes would otherwise
-//            take: 2,048 queries on 32,768 tokens at head_dim 64 49.3 ms there,
-//            0.96 ms (557 TFLOP/s) here; on 16,384 at 24 q / 8 kv heads of 128
-//            44.2 against 0.89 ms.  Dense tensors whose H * N is no multiple of
+//   kExactP  p * w enters PV as two bf16 operands, the upper half and what it
+//            left (p to 2^-16 relative at any magnitude), with the V-fog
+//            weights in fp32 and V unscaled, for the precision of the fp32
+//            VALU kernel (attn_generic_kernel) that these shapes would
+//            otherwise take; a key whose p is zero takes no part whatever its
+//            weight, and infinities in V and the weights carry through.  (V
+//            that is not finite still reaches the rows of the same query tile
+//            that a mask hides it from, as 0 * inf.)  fp16 keeps V as two
+//            bf16 tiles too (kSplitV): fp16 operands of p would share fp16's
+//            range, where a key 12 nats below the largest kept 8 bits, and one
+//            large weight took the digits of all others.  2,048 queries on
+//            32,768 tokens at head_dim 64 49.3 ms on the VALU kernel, bf16
+//            0.99 (fp16 1.09) here; on 16,384 at 24 q / 8 kv heads of 128 44.2
+//            against 0.64 (0.83).  Dense tensors whose H * N is no multiple of
 //            16 take it too (B=2, H=8, N=1,537, D=64, window 1,024: 722 us
-//            there, 39 us here; B=4, H=12, N=1,001, D=128, causal fog 2,035
-//            and 99 us);
+//            there, 40 us here; B=4, H=12, N=1,001, D=128, causal fog 2,035
+//            and 107 us);
 //   kSplit   grid z splits each query tile's key tiles (split s takes tiles
 //            s, s + S, ...); every split stores unnormalised partials (O,
 //            max, sum) merged by the combine kernel -- used when the chunks
@@ -72,17 +78,23 @@ constexpr int kPfWaves = 8;
 constexpr int kPfThreads = kPfWaves * 64;
 constexpr int kPfRows = kPfWaves * 32;  // query rows (position, head) per workgroup
 constexpr int kPfKT = 64;               // keys per tile (4 pages)
-constexpr int kPfStages = 4;            // LDS ring depth (a power of two)
+constexpr int kPfStages = 4;            // LDS ring depth (a power of two), but for kSplitV's K and V
 constexpr int kVRowW = kPfKT / 2 + 8;   // V^T tile row stride (32-bit words)
-// LDS geometry for head_dim D (128 or 64).
-template <int D>
+// LDS geometry for head_dim D (128 or 64).  kSplitV keeps V as two bf16 tiles
+// in the least rings that the loop allows: iteration t reads K of tile t + 1 and
+// V of tile t while it stores both of tile t + 2.
+template <int D, bool kSplitV>
 struct PfGeom {
+  static constexpr int kKStages = kSplitV ? 2 : kPfStages;
+  static constexpr int kVStages = kSplitV ? 3 : kPfStages;
   static constexpr int kKRow = D + 8;            // K tile row stride (elements)
   static constexpr int kKStage = kPfKT * kKRow;  // elements per K stage
-  static constexpr int kVStage = D * kVRowW;     // words per V^T stage
-  // K, V^T, bias; the exact-P instances also keep the tile's V weights and their largest magnitude.
+  static constexpr int kVTile = D * kVRowW;      // words per V^T tile
+  static constexpr int kVStage = kVTile * (kSplitV ? 2 : 1);
+  // K, V^T, bias; the exact-P instances also keep the tile's V weights.
   static constexpr size_t lds_bytes(bool exact_p) {
-    return (size_t)kPfStages * (kKStage * 2 + kVStage * 4 + kPfKT * 4 * (exact_p ? 2 : 1) + (exact_p ? 4 : 0));
+    return (size_t)kKStages * kKStage * 2 + (size_t)kVStages * kVStage * 4 +
+           (size_t)kPfStages * kPfKT * 4 * (exact_p ? 2 : 1);
   }
 };
 constexpr float kLog2e = 1.4426950408889634f;
@@ -138,15 +150,9 @@ __device__ __forceinline__ uint32_t pack2<f16_t>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
 }
 
-// The two halves of a packed dword, widened.
-template <typename T>
-__device__ __forceinline__ float unpack_lo(uint32_t w) {
-  return to_f32(__builtin_bit_cast(T, (uint16_t)w));
-}
-template <typename T>
-__device__ __forceinline__ float unpack_hi(uint32_t w) {
-  return to_f32(__builtin_bit_cast(T, (uint16_t)(w >> 16)));
-}
+// The two bf16 halves of a packed dword, widened.
+__device__ __forceinline__ float unpack_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float unpack_hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
 // max(a, b, c) in one instruction.  fmaxf on MFMA results first quiets each
 // input (one extra v_max per score); scores hold no signalling NaN, so the
@@ -173,13 +179,6 @@ __device__ __forceinline__ float max_xor32(float x) {
   return max3(a, b, b);
 }
 
-// max over the wave's lanes, in every lane (DPP within the rows of 16).
-__device__ __forceinline__ float wave_max(float x) {
-  x = row_max16(x);
-  auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l)); };
-  return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
-}
-
 // acc + lo + hi of two packed T values (one v_dot2 against (1, 1)).
 template <typename T>
 __device__ __forceinline__ float sum2(uint32_t w, float acc);
@@ -196,35 +195,42 @@ __device__ __forceinline__ float sum2<f16_t>(uint32_t w, float acc) {
 
 // Headroom of the lazy rescale, in log2 units: probabilities up to 2^8.
 constexpr float kRescaleSlack = 8.0f;
-// fp16 kExactP with V weights: p * w enters PV as fp16 operands, whose range
-// holds neither weights above 2^8 nor small ones to full precision.  The
-// exponentials' reference is therefore m_run + e_run, e_run an exponent of the
-// largest weight so far (within 2^kWRange of 1; raised when a tile's weights
-// exceed it by 2^kWSlack), which scales O and the softmax sum alike.
-constexpr int kWRange = 60;
-constexpr int kWSlack = 7;  // p * w < 2^(kRescaleSlack + kWSlack) = 2^15
+// a * b, and 0 where a is, whatever b (v_mul_legacy_f32).
+extern "C" __device__ float kessie_fmul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
+// The largest bf16 value.
+constexpr float kBf16Max = 3.38953139e38f;
+// Relative surplus of kExactP's p in PV (bf16), which keeps its second operand
+// from being zero beside a first that is not: both have p's sign, so that an
+// infinite V gives an infinity and not 0 * inf.  The softmax sum gets it too.
+constexpr float kPSurplus = 0x1p-20f;
 
 template <typename T, bool kBias, bool kVs, bool kSplit, int kMode, int kD, bool kExactP>
 __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   static_assert(kD == 128 || kD == 64, "head_dim 128 or 64");
   constexpr bool kDense = kMode == 1;
   constexpr bool kBig = kMode == 3;  // pages of 16 * 2^k tokens, k >= 1
-  constexpr int kKRow = PfGeom<kD>::kKRow;
-  constexpr int kKStage = PfGeom<kD>::kKStage;
-  constexpr int kVStage = PfGeom<kD>::kVStage;
+  constexpr bool kSplitV = kExactP && std::is_same<T, f16_t>::value;
+  typedef PfGeom<kD, kSplitV> Geom;
+  constexpr int kKRow = Geom::kKRow;
+  constexpr int kKStage = Geom::kKStage;
+  constexpr int kVStage = Geom::kVStage;
   constexpr int kDS = kD / 16;  // QK d-steps (B operand registers)
   constexpr int kDB = kD / 32;  // PV d-blocks (O accumulators)
   typedef typename Mma32<T>::v8 v8;
   typedef typename Mma32<T>::v4 v4;
+  typedef typename std::conditional<kExactP, bf16_t, T>::type PT;  // PV's operands
+  typedef typename Mma32<PT>::v8 p8;
   const int G = p.G;
   const int kPos = (unsigned)kPfRows / (unsigned)G;  // query positions per workgroup (rows past kPos * G idle)
   extern __shared__ __align__(16) unsigned char smem[];
-  T* ks = reinterpret_cast<T*>(smem);                                                // [stage][64][kKRow]
-  uint32_t* vts = reinterpret_cast<uint32_t*>(smem + (size_t)kPfStages * kKStage * 2);  // [stage][128][kVRowW]
-  float* fbs = reinterpret_cast<float*>(vts + kPfStages * kVStage);                   // [stage][64] bias*log2(e)
-  float* fws = fbs + kPfStages * kPfKT;                                               // [stage][64] V weights (kExactP)
-  float* fwm = fws + kPfStages * kPfKT;                                               // [stage] their max magnitude
-  constexpr bool kWExp = kExactP && kVs && std::is_same<T, f16_t>::value;
+  T* ks = reinterpret_cast<T*>(smem);                                                       // [stage][64][kKRow]
+  uint32_t* vts = reinterpret_cast<uint32_t*>(smem + (size_t)Geom::kKStages * kKStage * 2);  // [stage][kD][kVRowW]
+  float* fbs = reinterpret_cast<float*>(vts + Geom::kVStages * kVStage);                     // [stage][64] bias*log2(e)
+  float* fws = fbs + kPfStages * kPfKT;                                                      // [stage][64] V weights (kExactP)
+  auto k_stage = [&](int t) { return (t & (Geom::kKStages - 1)) * kKStage; };
+  auto v_stage = [&](int t) { return (kSplitV ? t % 3 : t & (kPfStages - 1)) * kVStage; };
+  auto f_stage = [&](int t) { return (t & (kPfStages - 1)) * kPfKT; };
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uniform(tid >> 6);
@@ -480,7 +486,9 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   const uint32_t pstride_b = (uint32_t)(p.page_stride * (int64_t)sizeof(T));
   auto page_span = [&](int pid, int first_tok, int64_t& off, int& bytes) {
     const int nrows = min(max(hi - first_tok, 0), 16);
-    const bool ok = (uint32_t)pid < n_ids && nrows > 0;
+    // (kExactP: a page wholly before the first key, which may hold anything, is not read either, as on the generic
+    // kernel: 0 * NaN.)
+    const bool ok = (uint32_t)pid < n_ids && nrows > 0 && (!kExactP || first_tok + 16 > lo);
     const uint32_t upid = ok ? (uint32_t)pid : 0u;
     uint64_t at = (uint64_t)upid * pstride_b;
     if constexpr (kBig)
@@ -538,48 +546,48 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   // probabilities stay unscaled and the softmax sum can be taken from them.
   // (kExactP: V stays as it is and the fp32 probabilities take the weights.)
   constexpr bool kScaleV = kVs && !kExactP;
-  auto store_weights = [&](int stage, int set) {
-    if (kVs && kExactP && tid < kPfKT) {  // wave 0
-      fws[stage * kPfKT + tid] = fk_r[set];
-      if constexpr (kWExp) fwm[stage] = wave_max(fabsf(fk_r[set]));
+  // (kSplitV: V is the sum of two bf16 values, exactly; an infinity is in the
+  // second one, which meets p's first operand only.)
+  auto store_v = [&](uint32_t* vd, int e, int set) {
+    const T a = vreg[set][0][e], b = vreg[set][1][e];
+    if constexpr (kSplitV) {
+      const float x = to_f32(a), y = to_f32(b);
+      const uint32_t h = pack2<bf16_t>(__builtin_amdgcn_fmed3f(x, -65504.0f, 65504.0f),
+                                       __builtin_amdgcn_fmed3f(y, -65504.0f, 65504.0f));
+      vd[(8 * kc + e) * kVRowW] = h;
+      vd[(8 * kc + e) * kVRowW + Geom::kVTile] = pack2<bf16_t>(x - unpack_lo(h), y - unpack_hi(h));
+    } else {
+      vd[(8 * kc + e) * kVRowW] =
+          kScaleV ? pack2<T>(to_f32(a) * fw0[set], to_f32(b) * fw1[set]) : bits16(a) | (bits16(b) << 16);
     }
   };
-  auto store = [&](int stage, int set) {
-    T* kd = ks + stage * kKStage + 8 * kc;
+  auto store_rows = [&](int t, int set) {  // tile t's K rows, bias and weights
+    T* kd = ks + k_stage(t) + 8 * kc;
 #pragma unroll
     for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
+    if (kBias && tid < kPfKT) fbs[f_stage(t) + tid] = fb_r[set] * kLog2e;
+    if (kVs && kExactP && tid < kPfKT) fws[f_stage(t) + tid] = fk_r[set];
+  };
+  const int v_at0 = 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
+  auto store = [&](int t, int set) {
+    store_rows(t, set);
     if (vload) {
-      uint32_t* vd = vts + stage * kVStage + 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        vd[(8 * kc + e) * kVRowW] = kScaleV ? pack2<T>(to_f32(vreg[set][0][e]) * fw0[set], to_f32(vreg[set][1][e]) * fw1[set])
-                                        : bits16(vreg[set][0][e]) | (bits16(vreg[set][1][e]) << 16);
+      for (int e = 0; e < 8; ++e) store_v(vts + v_stage(t) + v_at0, e, set);
     }
-    if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
-    store_weights(stage, set);
   };
 
   // Slice i of n (n >= 8) of store(): V^T word i for i < 8, then the K rows
   // and the bias at slice n-1 -- spread over the PV MFMAs.  With no tile
   // t+2 it rewrites a stage that no later tile reads.
-  auto store_slice = [&](int stage, int i, int n, int set) {
-    if (vload && i < 8) {
-      uint32_t* vd = vts + stage * kVStage + 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
-      vd[(8 * kc + i) * kVRowW] = kScaleV ? pack2<T>(to_f32(vreg[set][0][i]) * fw0[set], to_f32(vreg[set][1][i]) * fw1[set])
-                                      : bits16(vreg[set][0][i]) | (bits16(vreg[set][1][i]) << 16);
-    }
-    if (i == n - 1) {
-      T* kd = ks + stage * kKStage + 8 * kc;
-#pragma unroll
-      for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
-      if (kBias && tid < kPfKT) fbs[stage * kPfKT + tid] = fb_r[set] * kLog2e;
-      store_weights(stage, set);
-    }
+  auto store_slice = [&](int t, int i, int n, int set) {
+    if (vload && i < 8) store_v(vts + v_stage(t) + v_at0, i, set);
+    if (i == n - 1) store_rows(t, set);
   };
   // S^T of the tile in a stage: lane (col, half) reads K row 32kb + col.
   const T* kread = ks + col * kKRow + 8 * half;
-  auto qk = [&](int stage, f32x16 (&s)[2]) {
-    const T* kb0 = kread + stage * kKStage;
+  auto qk = [&](int t, f32x16 (&s)[2]) {
+    const T* kb0 = kread + k_stage(t);
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       s[kb] = f32x16{};
@@ -596,7 +604,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 #pragma unroll
   for (int i = 0; i < kDB; ++i) oacc[i] = f32x16{};
   float m_run = kNegInf, l_half = 0.0f;
-  float e_run = -(float)kWRange;  // (kWExp)
   const float c2 = p.sm_scale * kLog2e;
 
   // Tiles whose 64 keys all lie in [lo, hi) and are visible to every row of
@@ -629,9 +636,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   auto step = [&](int t, f32x16& c0, f32x16& c1, f32x16& x, int set) {
     auto sc = [&](int kb) -> f32x16& { return kb ? c1 : c0; };
     const int t0 = t_begin + t * kstep;
-    const int st_cur = t & (kPfStages - 1);
-    const int st_nxt = (t + 1) & (kPfStages - 1);
-    const int st_new = (t + 2) & (kPfStages - 1);
     // Tile t+3's global loads (none past the last tile: its ids are -1).
     const int pm3 = valid_mask(ids_a.ids);
     issue(t + 3, ids_a, set);
@@ -639,7 +643,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     ids_b = fetch_tile(t + 5);
 
     const bool interior = pm0 == 0xF && t >= ti_lo && t < ti_hi;
-    const float* fbt = fbs + st_cur * kPfKT + 8 * half;
+    const float* fbt = fbs + f_stage(t) + 8 * half;
     // Base-2 logits y = x * c2 (+ bias * log2 e); the tile max of y.
     if (!interior) {
       // This lane's keys of the tile form one interval of key offsets,
@@ -681,15 +685,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     // kRescaleSlack (log2 units); until then p = 2^(y - m_run) <= 2^kRescaleSlack,
     // as exact in T as any p <= 1, and the O accumulators are left alone.
     const float mnew = mloc > m_run + kRescaleSlack ? mloc : m_run;
-    float muse = mnew == kNegInf ? 0.0f : mnew;
-    float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
-    if constexpr (kWExp) {
-      const int we = ((int)(__builtin_bit_cast(uint32_t, fwm[st_cur]) >> 23) & 255) - 127;  // floor(log2), uniform
-      const float e_new = (float)we >= e_run + kWSlack ? (float)min(we, kWRange) : e_run;
-      alpha *= __builtin_amdgcn_exp2f(e_run - e_new);
-      muse += e_new;
-      e_run = e_new;
-    }
+    const float muse = mnew == kNegInf ? 0.0f : mnew;
+    const float alpha = mnew == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
     // (Rescaled before the exponentials, so that they, the next scores and PV
     // form one branch-free region.)
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
@@ -702,20 +699,34 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     // i+2, and a share of the VALU work -- one or two exponential pairs per
     // QK step, one slice of the stage store per PV step -- so the wave keeps
     // the matrix pipe busy while its VALU works.
-    constexpr int kQ = 2 * kDS;   // S^T MFMAs
-    constexpr int kPV = 4 * kDB;  // O^T MFMAs
-    constexpr int kPairsPer = 16 / kQ;
-    const T* kb0 = kread + st_nxt * kKStage;
-    const uint32_t* vr = vread + st_cur * kVStage;
+    // (kExactP at head_dim 128, whose probabilities' second operands have no
+    // registers left, runs as two halves of 32 keys: the QK steps of one score
+    // block with this half's exponentials, then the half's PV steps.  28-89
+    // VGPRs spilled otherwise; 2,048 bf16 queries on 16,384, 24 q / 8 kv, 746 ->
+    // 637 us, with V weights on 32-token pages 1,209 -> 789.  At head_dim 64,
+    // which spills nothing, it costs 3 %.)
+    constexpr int kHalves = kExactP && kD == 128 ? 2 : 1;
+    constexpr int kParts = kSplitV ? 2 : 1;
+    constexpr int kQ = 2 * kDS / kHalves;            // S^T steps of a half
+    constexpr int kPV = 4 * kDB * kParts / kHalves;  // V^T operands of a half
+    constexpr int kSteps = kHalves * (kQ + kPV);
+    constexpr int kPairsPer = 16 / (2 * kDS);
+    const T* kb0 = kread + k_stage(t + 1);
+    const uint32_t* vr = vread + v_stage(t);
+    // Step i: QK step (block, d-step) of the whole tile's 2 * kDS, or V^T operand of its 4 * kDB * kParts.
+    auto qk_step = [](int i) { return i % (kQ + kPV) < kQ ? i / (kQ + kPV) * kQ + i % (kQ + kPV) : -1; };
+    auto pv_step = [](int i) { return i / (kQ + kPV) * kPV + i % (kQ + kPV) - kQ; };
     auto op_read = [&](int i) {
-      if (i < kQ) return *reinterpret_cast<const v8*>(kb0 + 32 * (i < kDS ? 1 : 0) * kKRow + 16 * (i % kDS));
-      const int s = (i - kQ) / kDB, db = (i - kQ) % kDB;
-      return *reinterpret_cast<const v8*>(vr + 32 * db * kVRowW + 8 * (s ^ db));
+      const int q = qk_step(i);
+      if (q >= 0) return *reinterpret_cast<const v8*>(kb0 + 32 * (q < kDS ? 1 : 0) * kKRow + 16 * (q % kDS));
+      const int j = pv_step(i) / kParts, s = j / kDB, db = j % kDB, part = pv_step(i) % kParts;
+      return *reinterpret_cast<const v8*>(vr + part * Geom::kVTile + 32 * db * kVRowW + 8 * (s ^ db));
     };
     float ps0 = 0.0f, ps1 = 0.0f;  // the softmax sum, from p as rounded for PV
-    u32x4 pb[4];                   // p as the PV B operand, two keys per dword
-    u32x4 pl[4];                   // kExactP: what pb's rounding left of p, likewise
-    const float* fwt = fws + st_cur * kPfKT + 8 * half;
+    constexpr int kPRegs = 4 / kHalves;
+    u32x4 pb[kPRegs];              // p as the PV B operand, two keys per dword
+    u32x4 pl[kPRegs];              // kExactP: what pb left of p, likewise
+    const float* fwt = fws + f_stage(t) + 8 * half;
     auto exp_pair = [&](int j) {   // keys 2j, 2j+1 of this lane's 32
       const int kb = j >> 3, v = 2 * (j & 7);
       const float y0 = sc(kb)[v], y1 = sc(kb)[v + 1];
@@ -725,44 +736,56 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         ps0 += p0;
         ps1 += p1;
         if (kVs) {
-          p0 *= fwt[32 * kb + 16 * (v >> 3) + (v & 7)];
-          p1 *= fwt[32 * kb + 16 * (v >> 3) + (v & 7) + 1];
+          p0 = kessie_fmul_legacy(p0, fwt[32 * kb + 16 * (v >> 3) + (v & 7)]);
+          p1 = kessie_fmul_legacy(p1, fwt[32 * kb + 16 * (v >> 3) + (v & 7) + 1]);
         }
-        const uint32_t hi = pack2<T>(p0, p1);
-        pb[j >> 2][j & 3] = hi;
-        pl[j >> 2][j & 3] = pack2<T>(p0 - unpack_lo<T>(hi), p1 - unpack_hi<T>(hi));
+        // (An infinite p * w is infinite in the second operand only.)
+        const float h0 = kVs ? __builtin_amdgcn_fmed3f(p0, -kBf16Max, kBf16Max) : p0;
+        const float h1 = kVs ? __builtin_amdgcn_fmed3f(p1, -kBf16Max, kBf16Max) : p1;
+        if constexpr (kSplitV) {
+          const uint32_t hi = pack2<bf16_t>(h0, h1);
+          pb[(j >> 2) % kPRegs][j & 3] = hi;
+          pl[(j >> 2) % kPRegs][j & 3] = pack2<bf16_t>(p0 - unpack_lo(hi), p1 - unpack_hi(hi));
+        } else {
+          const uint32_t hi = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, h1), __builtin_bit_cast(uint32_t, h0), 0x07060302);
+          pb[(j >> 2) % kPRegs][j & 3] = hi;
+          pl[(j >> 2) % kPRegs][j & 3] = pack2<bf16_t>(fmaf(p0, 1.0f + kPSurplus, -unpack_lo(hi)), fmaf(p1, 1.0f + kPSurplus, -unpack_hi(hi)));
+        }
         return;
       }
       const uint32_t w = pack2<T>(p0, p1);
-      pb[j >> 2][j & 3] = w;
+      pb[(j >> 2) % kPRegs][j & 3] = w;
       if (j & 1)
         ps1 = sum2<T>(w, ps1);
       else
         ps0 = sum2<T>(w, ps0);
     };
-    v8 op[3];
-    op[0] = op_read(0);
-    op[1] = op_read(1);
+    constexpr int kOps = 3;
+    v8 op[kOps];
 #pragma unroll
-    for (int i = 0; i < kQ + kPV; ++i) {
-      if (i < kQ) {
+    for (int i = 0; i < kOps - 1; ++i) op[i] = op_read(i);
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+      const int q = qk_step(i);
+      if (q >= 0) {
         // The next tile's second block into x, then its first into c0
         // (whose exponentials, the first eight pairs, are issued by then).
-        if (i < kDS)
-          x = Mma32<T>::mma(op[i % 3], qv[i], i == 0 ? f32x16{} : x);
+        if (q < kDS)
+          x = Mma32<T>::mma(op[i % kOps], qv[q], q == 0 ? f32x16{} : x);
         else
-          c0 = Mma32<T>::mma(op[i % 3], qv[i - kDS], i == kDS ? f32x16{} : c0);
+          c0 = Mma32<T>::mma(op[i % kOps], qv[q - kDS], q == kDS ? f32x16{} : c0);
       } else {
-        const int s = (i - kQ) / kDB, db = (i - kQ) % kDB;
-        oacc[db] = Mma32<T>::mma(op[i % 3], __builtin_bit_cast(v8, pb[s]), oacc[db]);
-        if constexpr (kExactP) oacc[db] = Mma32<T>::mma(op[i % 3], __builtin_bit_cast(v8, pl[s]), oacc[db]);
+        const int j = pv_step(i) / kParts, s = j / kDB, db = j % kDB, part = pv_step(i) % kParts;
+        const p8 va = __builtin_bit_cast(p8, op[i % kOps]);
+        oacc[db] = Mma32<PT>::mma(va, __builtin_bit_cast(p8, pb[s % kPRegs]), oacc[db]);
+        if (kExactP && part == 0) oacc[db] = Mma32<PT>::mma(va, __builtin_bit_cast(p8, pl[s % kPRegs]), oacc[db]);
       }
-      if (i + 2 < kQ + kPV) op[(i + 2) % 3] = op_read(i + 2);
-      if (i < kQ) {
+      if (i + kOps - 1 < kSteps) op[(i + kOps - 1) % kOps] = op_read(i + kOps - 1);
+      if (q >= 0) {
 #pragma unroll
-        for (int j = 0; j < kPairsPer; ++j) exp_pair(i * kPairsPer + j);
+        for (int j = 0; j < kPairsPer; ++j) exp_pair(q * kPairsPer + j);
       } else {
-        store_slice(st_new, i - kQ, kPV, set ^ 1);
+        store_slice(t + 2, pv_step(i), kHalves * kPV, set ^ 1);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -791,6 +814,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
       qk(0, s0);
       sA = s0[0];
       sB = s0[1];
+      if (kSplitV) __syncthreads();  // (two K stages: iteration 0 stores over tile 0's)
     }
     // Unrolled by two so the score buffers alternate instead of being copied.
     // (Inside the prologue's branch, so the wait for the query loads stays
@@ -803,7 +827,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
   }
 
   // Lane (col, half) holds row frow at d = 32*db + 8*(v/4) + 4*half + (v%4).
-  const float l = l_half + __shfl_xor(l_half, 32);
+  float l = l_half + __shfl_xor(l_half, 32);
+  if (kExactP && !kSplitV) l += l * kPSurplus;
   // (A row before position 0 saw no key: it stores zeros, or an empty partial.)
   if (qi > qi_last) return;
   if (kSplit && part_out) {
@@ -819,7 +844,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
         *reinterpret_cast<f32x4*>(dst + 32 * db + 8 * vq) =
             f32x4{oacc[db][4 * vq], oacc[db][4 * vq + 1], oacc[db][4 * vq + 2], oacc[db][4 * vq + 3]};
     if (half == 0) {
-      p.ws_m[r] = m_run == kNegInf ? kNegInf : (kWExp ? m_run + e_run : m_run) * kLn2;
+      p.ws_m[r] = m_run == kNegInf ? kNegInf : m_run * kLn2;
       p.ws_l[r] = l;
     }
     return;
@@ -840,7 +865,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
 template <typename T, bool kBias, bool kVs, bool kSplit, int kMode, int kD, bool kExactP>
 int launch_one(const Params& p, dim3 grid, hipStream_t stream) {
   static bool lds_set[64] = {};  // per instance and device
-  constexpr size_t lds = PfGeom<kD>::lds_bytes(kExactP);
+  constexpr size_t lds = PfGeom<kD, kExactP && std::is_same<T, f16_t>::value>::lds_bytes(kExactP);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   const void* fn = reinterpret_cast<const void*>(prefill_mfma_kernel<T, kBias, kVs, kSplit, kMode, kD, kExactP>);

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from oracle.attention import fused_fog_attention_ref, windowed_attention_ref
+from tests.exact64 import attend64, close_to_rounding
 from tests.inputs import gen
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,22 @@ def test_dense_ragged(dev, monkeypatch, b, h, n, d, splits, window, causal, fog)
     err = (out.double().cpu() - ref.double()).norm()
     rounding = (ref.half().double() - ref.double()).norm()
     assert err <= 1.02 * rounding + 2e-5 * ref.double().norm(), f"error {err:.3e}, rounding alone {rounding:.3e}"
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_dense_ragged_one_large_weight(dev, monkeypatch, d, splits):
+    """A fog weight of 2^16 on a key that few rows see, beside weights of 1: the rows that do not see it keep their
+    precision."""
+    from kessie_amd.kessie_hip_ctypes import KeSSieKernels
+
+    monkeypatch.setenv("KESSIE_DENSE_SPLITS", str(splits))
+    h, n = 3, 517
+    q, k, v = [torch.randn(1, h, n, d, generator=gen(dev, 90 + i), device=dev).half() for i in range(3)]
+    w = torch.ones(n, device=dev)
+    w[400] = 2.0 ** 16
+    v[:, :, 400] *= 2.0 ** -10
+    out = KeSSieKernels().fused_fog_attention(q, k, v, w, window_size=64, causal=True)
+    ref = attend64(q[0].transpose(0, 1), k[0].transpose(0, 1), v[0].transpose(0, 1), 0, w, None, 64)
+    for r in range(n):
+        close_to_rounding(out[0, :, r], ref[r], torch.float16)

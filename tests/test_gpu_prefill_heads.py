@@ -1,9 +1,9 @@
 """GPU parity of chunked prefill on head_dim 64 and on GQA ratios that are no
-power of two: MFMA instances whose probabilities keep fp32 precision.
+power of two: MFMA instances whose probabilities enter PV as two bf16 operands.
 
-Tolerance: the kernel's own error is that of fp32 sums (2e-5 of the result's
-norm, far above 2^-16 per probability), so the distance from the oracle is that
-of rounding the oracle's result to the type, and no more."""
+Tolerance: the kernel's own error is that of fp32 sums and of probabilities to
+2^-16 (2e-5 of the result's norm), so the distance from the oracle is that of
+rounding the oracle's result to the type, and no more."""
 import pytest
 import torch
 
@@ -134,3 +134,111 @@ def test_prefill_large_common_bias(dev, hq, hkv, d):
     pool, table, lens = paged(k, v)
     out = ops.fog_prefill(q, pool, table, lens, n, fog_bias=bias)
     close_to_rounding(out[0], attend64(q[0], k, v, n - c), torch.float16, own=1.4e-3)
+
+
+SHAPES = pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (6, 2, 128)])
+
+
+def _kvq(dev, n, c, hq, hkv, d, dtype, seed):
+    k, v = (torch.randn(n, hkv, d, generator=gen(dev, seed + i), device=dev).to(dtype) for i in (0, 1))
+    return k, v, torch.randn(c, hq, d, generator=gen(dev, seed + 2), device=dev).to(dtype)
+
+
+@SHAPES
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+def test_prefill_small_probabilities(dev, monkeypatch, hq, hkv, d, dt):
+    """One key 12 above all others, with a small V (an attention sink): the result rests on probabilities of e^-12,
+    which 16-bit operands of fp16's range hold to a part in 1,000 only."""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", "1")
+    dtype, n, c = DT[dt], 4096, 70
+    k = torch.zeros(n, hkv, d, device=dev, dtype=dtype)
+    k[5] = 12 / d ** 0.5
+    v = (1 + 0.1 * torch.randn(n, hkv, d, generator=gen(dev, 61), device=dev)).to(dtype)
+    v[5] = 2.0 ** -10
+    q = torch.ones(c, hq, d, device=dev, dtype=dtype)
+    pool, table, lens = paged(k, v)
+    close_to_rounding(ops.fog_prefill(q[None], pool, table, lens, n)[0], attend64(q, k, v, n - c), dtype)
+
+
+@SHAPES
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("where", ["faint", "window", "future"])
+def test_prefill_fp16_one_large_weight(dev, monkeypatch, hq, hkv, d, splits, where):
+    """A weight of 2^16 on a key whose probability is negligible, or that the window or the causal mask hides from
+    some rows, costs those rows' other keys nothing."""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
+    n, c, window, at = 700, 64, 0, 190
+    if where == "window":
+        window, at = 100, 569  # the chunk's first 32 rows see it
+    elif where == "future":
+        at = 690  # the last ten rows see it, in the others' tile
+    k, v, q = _kvq(dev, n, c, hq, hkv, d, torch.float16, 71)
+    w, bias = torch.ones(n, device=dev), torch.zeros(n, device=dev)
+    w[at] = 2.0 ** 16
+    v[at] *= 2.0 ** -10  # (results of the rows that see it stay in fp16's range)
+    if where == "faint":
+        bias[at] = -60.0
+    pool, table, lens = paged(k, v)
+    out = ops.fog_prefill(q[None], pool, table, lens, n, fog_vscale=w, fog_bias=bias, window=window)[0]
+    ref = attend64(q, k, v, n - c, w, bias, window)
+    for r in range(c):
+        close_to_rounding(out[r], ref[r], torch.float16)
+
+
+@SHAPES
+@pytest.mark.parametrize("splits", [1, 3])
+def test_prefill_fp16_weights_under_a_mask(dev, monkeypatch, hq, hkv, d, splits):
+    """Every key under a mask of -1e9: key tiles and splits, whose weights differ, still count alike."""
+    from kessie_amd import ops
+
+    monkeypatch.setenv("KESSIE_PREFILL_SPLITS", str(splits))
+    n, c = 1000, 40
+    k, v, q = _kvq(dev, n, c, hq, hkv, d, torch.float16, 75)
+    k.zero_()
+    w, bias = torch.logspace(-4, 0, n, device=dev), torch.full((n,), -1e9, device=dev)
+    pool, table, lens = paged(k, v)
+    out = ops.fog_prefill(q[None], pool, table, lens, n, fog_vscale=w, fog_bias=bias)[0]
+    close_to_rounding(out, attend64(q, k, v, n - c, w, bias), torch.float16)
+
+
+@SHAPES
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("what", ["v", "-v", "weight", "hidden weight"])
+def test_prefill_infinities(dev, hq, hkv, d, dt, what):
+    """An infinity in V or in a weight shows as an infinity where its key takes part, and an infinite weight not at
+    all where the probability is zero."""
+    from kessie_amd import ops
+
+    dtype, n, c = DT[dt], 300, 60
+    k, v, q = _kvq(dev, n, c, hq, hkv, d, dtype, 78)
+    w, bias = torch.ones(n, device=dev), torch.zeros(n, device=dev)
+    if what.endswith("v"):
+        v[130, :, 3] = float("-inf" if what == "-v" else "inf")
+    else:
+        w[130] = float("inf")
+        if what == "hidden weight":
+            bias[130] = -float("inf")
+    pool, table, lens = paged(k, v)
+    out = ops.fog_prefill(q[None], pool, table, lens, n, fog_vscale=w, fog_bias=bias)[0].double().cpu()
+    ref = attend64(q, k, v, n - c, w, bias)
+    finite = ref.isfinite()
+    assert finite.all() == (what == "hidden weight") and not ref.isnan().any()
+    assert torch.equal(out[~finite], ref[~finite])
+    close_to_rounding(torch.where(finite, out, 0.0), torch.where(finite, ref, 0.0), dtype)
+
+
+@SHAPES
+def test_prefill_pages_before_the_window(dev, hq, hkv, d):
+    """Pages wholly before the window may be anyone's, also where the first key tile covers them."""
+    from kessie_amd import ops
+
+    n, c, window = 300, 20, 40  # keys from 241 on; the tile begins at 192
+    k, v, q = _kvq(dev, n, c, hq, hkv, d, torch.bfloat16, 82)
+    pool, table, lens = paged(k, v)
+    pool[:15] = float("nan")
+    out = ops.fog_prefill(q[None], pool, table, lens, n, window=window)[0]
+    close_to_rounding(out, attend64(q, k, v, n - c, window=window), torch.bfloat16)
