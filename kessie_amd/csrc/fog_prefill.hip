@@ -198,6 +198,13 @@ constexpr float kRescaleSlack = 8.0f;
 // a * b, and 0 where a is, whatever b (v_mul_legacy_f32).
 extern "C" __device__ float kessie_fmul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
 
+// A bias in base 2.  A finite one stays finite: masks of the type's lowest value
+// hide keys alike, also where they hide all of a row's.
+constexpr float kF32Max = 3.402823466e38f;
+__device__ __forceinline__ float base2_bias(float b) {
+  return fabsf(b) <= kF32Max ? fmaxf(fminf(b * kLog2e, kF32Max), -kF32Max) : b;
+}
+
 // The largest bf16 value.
 constexpr float kBf16Max = 3.38953139e38f;
 // Relative surplus of kExactP's p in PV (bf16), which keeps its second operand
@@ -565,7 +572,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     T* kd = ks + k_stage(t) + 8 * kc;
 #pragma unroll
     for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
-    if (kBias && tid < kPfKT) fbs[f_stage(t) + tid] = fb_r[set] * kLog2e;
+    if (kBias && tid < kPfKT) fbs[f_stage(t) + tid] = base2_bias(fb_r[set]);
     if (kVs && kExactP && tid < kPfKT) fws[f_stage(t) + tid] = fk_r[set];
   };
   const int v_at0 = 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);

@@ -101,7 +101,8 @@ def test_prefill_fp16_weights_of_any_magnitude(dev, monkeypatch, hq, hkv, d, spl
 
 
 @pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (8, 2, 128), (6, 2, 128)])
-@pytest.mark.parametrize("low", [-1e38, -1e9, -65504.0, -float("inf")])
+@pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, torch.finfo(torch.bfloat16).min, -1e38, -1e9, -65504.0,
+                                 -float("inf")])
 @pytest.mark.parametrize("splits", [1, 2])
 def test_prefill_bias_masks(dev, monkeypatch, hq, hkv, d, low, splits):
     """Keys hidden by the lowest values a mask holds, and with the finite ones a sequence whose keys are all hidden
@@ -113,7 +114,7 @@ def test_prefill_bias_masks(dev, monkeypatch, hq, hkv, d, low, splits):
     q = randn((2, 70, hq, d), torch.bfloat16, dev, 20)
     bias = fog_bias(300, 0.5, 0.5, {3}, 0.1).to(dev).repeat(2, 1)
     bias[0, 5:100] = low
-    if low in (-1e38, -1e9):  # (fp32 spacing there is above any score: all keys alike)
+    if -float("inf") < low < -65504.0:  # (fp32 spacing there is above any score: all keys alike)
         bias[1] = low
     out = ops.fog_prefill(q, pool, table, lens, 300, fog_bias=bias)
     ref = paged_prefill_ref(q.cpu(), pool.cpu(), table.cpu(), lens.cpu(), None, bias.cpu(), 0)
