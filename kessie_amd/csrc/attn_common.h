@@ -95,6 +95,13 @@ __device__ __forceinline__ bool key_visible(int q_pos, int t, int window, int ca
   return true;
 }
 
+// MFMA prefill shapes that take kExactP (fog_prefill.hip), which the generic
+// kernel served before: paged head_dim 64, GQA ratios that are no power of two,
+// and the dense tensors that ask for it.
+inline bool prefill_exact_p(const Params& p) {
+  return p.page_table != nullptr ? p.D == 64 || (p.G & (p.G - 1)) != 0 : p.dense_exact_p != 0;
+}
+
 // Row index into the partial workspace / output for (b, i, h).
 __device__ __forceinline__ int64_t row_id(const Params& p, int b, int i, int h) {
   return ((int64_t)b * p.C + i) * p.Hq + h;

@@ -2130,6 +2130,19 @@ static int run_prefill_mfma(kessie::attn::Params& p, int dtype, void* workspace,
   using namespace kessie;
   using namespace kessie::attn;
   p.num_splits = prefill_mfma_splits(p.B, p.C, p.Hkv, p.G, p.max_ctx, p.causal != 0);
+  if (prefill_exact_p(p) && p.q_start == nullptr) {
+    // Shapes of kessie_fog_prefill_paged that ran on the generic kernel before are refused by its need for a
+    // workspace, as they were, and split no further than the workspace holds.
+    const int64_t rows = (int64_t)p.B * p.C * p.Hq;
+    const int g = prefill_splits(p.B, p.C, p.Hkv, p.G, p.max_ctx, p.page_size);
+    const size_t need = g > 1 ? partial_bytes(rows, g, p.D) : 0;
+    KESSIE_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need), KESSIE_ERR_WORKSPACE,
+                   "fog prefill: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+    KESSIE_REQUIRE(need == 0 || aligned16(workspace), KESSIE_ERR_INVALID,
+                   "fog prefill: workspace not 16-byte aligned");
+    const bool usable = workspace != nullptr && aligned16(workspace);
+    while (p.num_splits > 1 && !(usable && partial_bytes(rows, p.num_splits, p.D) <= workspace_bytes)) --p.num_splits;
+  }
   p.direct_out = p.num_splits == 1 ? 1 : 0;
   p.launch_combine = 0;
   // Longest query tiles first when the causal triangle dominates (the chunk is

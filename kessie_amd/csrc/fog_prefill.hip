@@ -921,13 +921,6 @@ int launch_mode(const Params& p, dim3 grid, hipStream_t stream) {
   return KESSIE_ERR_UNSUPPORTED;
 }
 
-// Shapes whose probabilities are kept to fp32 precision (kernel header): paged
-// head_dim 64, GQA ratios that are no power of two, and the dense tensors that
-// ask for it.
-bool prefill_exact_p(const Params& p) {
-  return p.page_table != nullptr ? p.D == 64 || (p.G & (p.G - 1)) != 0 : p.dense_exact_p != 0;
-}
-
 template <typename T>
 int launch_prefill(Params& p, hipStream_t stream) {
   const int kpos = kPfRows / p.G;

@@ -243,3 +243,19 @@ def test_prefill_pages_before_the_window(dev, hq, hkv, d):
     pool[:15] = float("nan")
     out = ops.fog_prefill(q[None], pool, table, lens, n, window=window)[0]
     close_to_rounding(out, attend64(q, k, v, n - c, window=window), torch.bfloat16)
+
+
+def test_prefill_small_workspace(dev):
+    """A workspace that the generic kernel, which ran head_dim 64 before, does without or is refused for."""
+    from kessie_amd import ops
+
+    tiny = torch.empty(16, dtype=torch.uint8, device=dev)
+    for c, n, refused in ((512, 4096, False), (64, 512, True)):
+        k, v, q = _kvq(dev, n, c, 32, 8, 64, torch.bfloat16, 85)
+        pool, table, lens = paged(k, v)
+        if refused:
+            with pytest.raises(RuntimeError, match="workspace"):
+                ops.fog_prefill(q[None], pool, table, lens, n, ws=tiny)
+        else:
+            out = ops.fog_prefill(q[None], pool, table, lens, n, ws=tiny)
+            close_to_rounding(out[0, :40], attend64(q[:40], k[:n - c + 40], v[:n - c + 40], n - c), torch.bfloat16)
