@@ -1436,6 +1436,13 @@ int prefill_splits(int B, int C, int Hkv, int G, int max_ctx, int page_size) {
 
 template <typename T>
 int launch_generic(Params& p, hipStream_t stream) {
+  // Testing switch: KESSIE_REQUIRE_MFMA=1 makes a call that would run here an
+  // error (the tests use it to show which route ran).
+  if (env_int("KESSIE_REQUIRE_MFMA", 0)) {
+    set_error(KESSIE_ERR_UNSUPPORTED, "fog attention: B=%d C=%d Hq=%d Hkv=%d D=%d runs on the generic kernel", p.B, p.C,
+              p.Hq, p.Hkv, p.D);
+    return KESSIE_ERR_UNSUPPORTED;
+  }
   const int tiles = div_up(p.C * p.G, kGenRT);
   const size_t lds = generic_lds_bytes(p.D);
   if (lds > 48 * 1024) {
@@ -2480,43 +2487,32 @@ static void dense_fp16(const void* Q, const void* K, const void* V, void* O, con
   // that took them before (B=2, H=8, N=1,537, D=64, window 1,024: 722 us
   // there, 39 us here).
   const bool ragged = ((int64_t)H * N) % 16 != 0;
-  // Testing switch: KESSIE_REQUIRE_MFMA=1 makes a shape that is not on the
-  // rounded-probability route an error (the tests use it to show which route
-  // ran).
-  const bool require = env_int("KESSIE_REQUIRE_MFMA", 0) != 0;
   Params m = p;
   m.page_size = 16;
   m.page_stride = 16 * (int64_t)D;
   m.num_pages = div_up(N, 16);
   m.dense_exact_p = ragged ? 1 : 0;
-  if (!(require && ragged)) {
-    if (prefill_mfma_ok(m, KESSIE_DTYPE_F16)) {
-      const hipStream_t s = as_stream(stream);
-      int split_q0 = 0;
-      const int S = dense_splits(B, H, N, window, causal, &split_q0);
-      const int64_t rows = (int64_t)B * (N - split_q0) * H;  // partial rows: the split tiles' queries
-      const size_t need = partial_bytes(rows, S, D);
-      void* ws = S > 1 && need <= ((size_t)1 << 30) ? dense_workspace(need, s) : nullptr;
-      if (ws != nullptr) {
-        m.num_splits = S;
-        m.split_q0 = split_q0;
-        m.direct_out = 0;
-        carve_workspace(m, ws, rows);
-        if (prefill_mfma(m, KESSIE_DTYPE_F16, s) != KESSIE_OK) return;  // error recorded
-        Params c = m;  // the combine's rows: positions split_q0 .. N-1
-        c.C = N - split_q0;
-        c.q0_off = split_q0;
-        launch_combine<f16_t>(c, rows, s);
-        check_launch("dense attention (combine)");
-        return;
-      }
-      prefill_mfma(m, KESSIE_DTYPE_F16, s);  // records any launch error
+  if (prefill_mfma_ok(m, KESSIE_DTYPE_F16)) {
+    const hipStream_t s = as_stream(stream);
+    int split_q0 = 0;
+    const int S = dense_splits(B, H, N, window, causal, &split_q0);
+    const int64_t rows = (int64_t)B * (N - split_q0) * H;  // partial rows: the split tiles' queries
+    const size_t need = partial_bytes(rows, S, D);
+    void* ws = S > 1 && need <= ((size_t)1 << 30) ? dense_workspace(need, s) : nullptr;
+    if (ws != nullptr) {
+      m.num_splits = S;
+      m.split_q0 = split_q0;
+      m.direct_out = 0;
+      carve_workspace(m, ws, rows);
+      if (prefill_mfma(m, KESSIE_DTYPE_F16, s) != KESSIE_OK) return;  // error recorded
+      Params c = m;  // the combine's rows: positions split_q0 .. N-1
+      c.C = N - split_q0;
+      c.q0_off = split_q0;
+      launch_combine<f16_t>(c, rows, s);
+      check_launch("dense attention (combine)");
       return;
     }
-  }
-  if (require) {
-    set_error(KESSIE_ERR_UNSUPPORTED, "dense attention: B=%d H=%d N=%d D=%d runs at the generic kernel's precision", B,
-              H, N, D);
+    prefill_mfma(m, KESSIE_DTYPE_F16, s);  // records any launch error
     return;
   }
   launch_generic<f16_t>(p, as_stream(stream));

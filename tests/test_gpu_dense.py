@@ -1,9 +1,8 @@
 """GPU parity: the reference's dense launchers (launch_kessie_windowed_attn,
 launch_kessie_fused_fog_attn: fp16 [B, H, N, D], every position a query)
 through KeSSieKernels vs the CPU oracle (fp32 on upcast inputs).  head_dim 128
-or 64 with H*N a multiple of 16 runs on the MFMA prefill kernel (table-less
-pages), other shapes on the generic kernel.  Tolerance |gpu - ref| <= 2e-2 +
-1e-2*|ref|."""
+or 64 runs on the MFMA prefill kernel (table-less pages), misaligned tensors on
+the generic kernel.  Tolerance |gpu - ref| <= 2e-2 + 1e-2*|ref|."""
 import pytest
 import torch
 
@@ -24,13 +23,11 @@ def _qkv(dev, b, h, n, d, seed):
     return [torch.randn(b, h, n, d, generator=gen(dev, seed + i), device=dev).to(torch.float16) for i in range(3)]
 
 
-# MFMA route: D = 128 or 64 and H*N a multiple of 16 (N itself need not be:
-# the last page of every head ends inside it); the rest (here (2, 2, 100, *)
-# and (1, 3, 50, 64)) run on the generic kernel.
+# Every shape is on the MFMA route: the last page of a head may end inside it,
+# and H*N need not be a multiple of 16 (here (2, 2, 100, *) and (1, 3, 50, 64)).
 SHAPES = [(2, 4, 256, 128), (1, 3, 1024, 128), (2, 32, 100, 128), (1, 4, 1000, 128), (3, 16, 37, 128),
           (2, 2, 100, 128), (2, 3, 64, 64), (1, 2, 48, 64), (2, 4, 256, 64), (1, 4, 1000, 64), (3, 16, 37, 64),
           (2, 2, 100, 64), (1, 3, 50, 64)]
-MFMA_ROUTE = {s for s in SHAPES if (s[1] * s[2]) % 16 == 0}
 
 
 @pytest.mark.parametrize("b,h,n,d", SHAPES)
@@ -38,8 +35,7 @@ MFMA_ROUTE = {s for s in SHAPES if (s[1] * s[2]) % 16 == 0}
 def test_windowed_attention(dev, monkeypatch, b, h, n, d, window, causal):
     from kessie_amd.kessie_hip_ctypes import KeSSieKernels
 
-    if (b, h, n, d) in MFMA_ROUTE:
-        monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")  # the launcher errors if it would use the generic kernel
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")  # the launcher errors if it would use the generic kernel
     q, k, v = _qkv(dev, b, h, n, d, seed=n + d + window)
     out = KeSSieKernels().windowed_attention(q, k, v, window_size=window, causal=causal)
     ref = windowed_attention_ref(q.float().cpu(), k.float().cpu(), v.float().cpu(), window, causal)
@@ -51,8 +47,7 @@ def test_windowed_attention(dev, monkeypatch, b, h, n, d, window, causal):
 def test_fused_fog_attention(dev, monkeypatch, b, h, n, d, window):
     from kessie_amd.kessie_hip_ctypes import KeSSieKernels
 
-    if (b, h, n, d) in MFMA_ROUTE:
-        monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
     q, k, v = _qkv(dev, b, h, n, d, seed=2 * n + d)
     w = torch.rand(n, generator=gen(dev, 7), device=dev)
     out = KeSSieKernels().fused_fog_attention(q, k, v, w, window_size=window)
@@ -81,15 +76,32 @@ def test_dense_mfma_matches_generic(dev, monkeypatch, d):
 
 
 def test_require_mfma_switch_rejects_a_generic_shape(dev, monkeypatch):
-    """H*N not a multiple of 16 has no MFMA route: with the switch set the
-    launcher reports it instead of running the generic kernel."""
+    """Tensors off a 16-byte boundary have no MFMA route: with the switch set
+    the launcher reports it, without it the generic kernel runs."""
     from kessie_amd import _lib
     from kessie_amd.kessie_hip_ctypes import KeSSieKernels
 
-    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
     q, k, v = _qkv(dev, 1, 3, 50, 64, seed=13)
+    off = torch.empty(q.numel() + 1, dtype=torch.float16, device=dev)[1:].view(q.shape).copy_(q)
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
     with pytest.raises(_lib.KeSSieError, match="generic kernel"):
-        KeSSieKernels().windowed_attention(q, k, v)
+        KeSSieKernels().windowed_attention(off, k, v)
+    monkeypatch.delenv("KESSIE_REQUIRE_MFMA")
+    _check(KeSSieKernels().windowed_attention(off, k, v),
+           windowed_attention_ref(q.float().cpu(), k.float().cpu(), v.float().cpu()))
+
+
+def test_require_mfma_switch_on_paged_calls(dev, monkeypatch):
+    """The paged decode and prefill report a shape of the generic kernel (12-token pages) likewise."""
+    from kessie_amd import _lib, ops
+    from tests.inputs import decode_case
+
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
+    q, pool, table, lens = decode_case(1, 8, 2, 64, 60, 12, torch.float16, dev, seed=14)
+    with pytest.raises(_lib.KeSSieError, match="generic kernel"):
+        ops.fog_decode(q, pool, table, lens, 60)
+    with pytest.raises(_lib.KeSSieError, match="generic kernel"):
+        ops.fog_prefill(q[:, None], pool, table, lens, 60)
 
 
 @pytest.mark.parametrize("n", [512, 2048, 4096])

@@ -14,6 +14,12 @@ from tests.inputs import gen
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def mfma_only(monkeypatch):
+    """A call that would run on the generic kernel is an error in this file."""
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
+
+
 @pytest.mark.parametrize("b,h,n,d,splits", [
     (1, 1, 1, 64, 0), (1, 1, 1, 128, 0),        # one key
     (3, 1, 15, 64, 0), (2, 5, 17, 128, 0),      # around a page

@@ -14,6 +14,12 @@ from tests.inputs import decode_case, gen, randn
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def mfma_only(monkeypatch):
+    """A call that would run on the generic kernel is an error in this file."""
+    monkeypatch.setenv("KESSIE_REQUIRE_MFMA", "1")
+
 DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
 
 
