@@ -214,8 +214,8 @@ class _FogCache:
         builds (in ``dtype``, widened to fp32) for that sequence's own kv_len =
         seq_lens[b], zero past it.  One launch on the current stream, no host
         synchronisation.  Shared by the layers of a step when the lengths are
-        known on the host (``seq_lens_host``): cached per generation and length
-        tuple; without them it is recomputed on every call.
+        known on the host (``seq_lens_host``, a tuple or a tensor): cached per
+        generation and length tuple; without them it is recomputed on every call.
 
         Under HIP graph capture the fill is always recorded (a cached view
         would leave the graph without it, replaying whatever an eager call
@@ -227,7 +227,9 @@ class _FogCache:
         capturing = torch.device(device).type == "cuda" and torch.cuda.is_current_stream_capturing()
         key = None
         if seq_lens_host is not None and not capturing:
-            key = (state["generation"], kv_len, str(device), dtype, tuple(int(x) for x in seq_lens_host.tolist()))
+            if not isinstance(seq_lens_host, tuple):
+                seq_lens_host = tuple(int(x) for x in seq_lens_host.tolist())
+            key = (state["generation"], kv_len, str(device), dtype, seq_lens_host)
             cached = self._rows_cache  # (key, view), replaced as one attribute
             if cached is not None and cached[0] == key:
                 return cached[1]
@@ -463,6 +465,20 @@ class KeSSieAttentionImpl:
             cls._split_cache = (key, val)
         return val
 
+    # (key, sum) of the last _seen, replaced as one attribute like _split_cache.
+    _seen_cache = None
+
+    @classmethod
+    def _seen(cls, lens, lo, hi, most):
+        """Sum of min(n, most) over lens[lo:hi], once a step: the layers repeat the content that keys it."""
+        key = (lens, lo, hi, most)
+        cached = cls._seen_cache
+        if cached is not None and cached[0] == key:
+            return cached[1]
+        val = sum(min(n, most) for n in lens[lo:hi])
+        cls._seen_cache = (key, val)
+        return val
+
     def _attend(self, args, kwargs, state):
         from . import ops
 
@@ -501,20 +517,23 @@ class KeSSieAttentionImpl:
         # Fog bias per sequence (row b built for that sequence's own length),
         # rows read with a batch stride by the kernels.
         bias = None
-        lens_host = None
+        lens_host = None  # read with the fog on only, which needs them for its rows: 2 us a layer otherwise
         if state is not None and kv_len > 0 and nseq > 0:
             lens_host = getattr(meta, "seq_lens_cpu", None)
-            bias = _FOG_CACHE.get_fog_bias_rows(lens, kv_len, query.device, query.dtype, state,
-                                                lens_host[:nseq] if lens_host is not None else None)
+            if lens_host is not None:
+                lens_host = tuple(lens_host[:nseq].tolist())
+            bias = _FOG_CACHE.get_fog_bias_rows(lens, kv_len, query.device, query.dtype, state, lens_host)
 
         if decode:
             if decode == list(range(decode[0], decode[0] + len(decode))):
                 lo, hi = decode[0], decode[-1] + 1
                 q_dec = q[qsl[lo]:qsl[lo] + (hi - lo)]
                 seen = 0  # tokens the decode rows see, where the host knows them
-                if lens_host is not None and hi - lo > 1:
-                    w = self.window or kv_len
-                    seen = sum(min(n, w) for n in lens_host[lo:hi].tolist())
+                most = min(self.window or kv_len, kv_len)
+                # (It can matter from 24 MiB of K/V on, where the balanced split has that much to save.)
+                if lens_host is not None and hi - lo > 1 and (
+                        (hi - lo) * most * 2 * self.num_kv_heads * d * query.element_size() >= 24 << 20):
+                    seen = self._seen(lens_host, lo, hi, most)
                 ops.fog_decode(q_dec, kv_cache, table[lo:hi], lens[lo:hi], kv_len,
                                fog_bias=None if bias is None else bias[lo:hi],
                                window=self.window, sm_scale=self.scale, layout=layout,

@@ -200,11 +200,18 @@ def fog_decode(q: torch.Tensor, pool: torch.Tensor, page_table: torch.Tensor, ct
     if ws is None:
         ws = workspace(need, q.device, "attn")
     wsz = 0 if ws is None else ws.numel() * ws.element_size()
-    _lib.check("kessie_fog_decode_batch", lib.kessie_fog_decode_batch(
+    if seen_total:
+        _lib.check("kessie_fog_decode_batch", lib.kessie_fog_decode_batch(
+            _ptr(q), C.c_void_p(pv.k_ptr), pv.num_pages, pv.page_stride, pv.tok_stride, pv.kv_stride,
+            pv.head_stride, _ptr(page_table), page_table.stride(0), _ptr(ctx_lens), _ptr(vs), vs_bs,
+            _ptr(bi), bi_bs, _ptr(out), b, hq, pv.num_kv_heads, d, pv.page_size, int(max_ctx), int(window),
+            float(sm_scale), dt, int(seen_total), _ptr(ws), wsz, _stream_ptr(stream, q.device)))
+        return out
+    _lib.check("kessie_fog_decode_paged", lib.kessie_fog_decode_paged(
         _ptr(q), C.c_void_p(pv.k_ptr), pv.num_pages, pv.page_stride, pv.tok_stride, pv.kv_stride,
         pv.head_stride, _ptr(page_table), page_table.stride(0), _ptr(ctx_lens), _ptr(vs), vs_bs,
         _ptr(bi), bi_bs, _ptr(out), b, hq, pv.num_kv_heads, d, pv.page_size, int(max_ctx), int(window),
-        float(sm_scale), dt, int(seen_total), _ptr(ws), wsz, _stream_ptr(stream, q.device)))
+        float(sm_scale), dt, _ptr(ws), wsz, _stream_ptr(stream, q.device)))
     return out
 
 
@@ -312,8 +319,8 @@ def fog_prefill_varlen(q: torch.Tensor, query_start_loc: torch.Tensor, max_query
     take (the caller then runs fog_prefill per sequence).  ws: split-K
     workspace (a cached one when None), used when the chunks are too few to
     fill the device."""
-    return _prefill_varlen("kessie_fog_prefill_varlen", q, query_start_loc, max_query_len, pool, page_table, ctx_lens,
-                           max_ctx, fog_vscale, fog_bias, window, causal, sm_scale, layout, out, ws, stream)
+    return fog_prefill_batch(q, query_start_loc, max_query_len, pool, page_table, ctx_lens, max_ctx, fog_vscale, fog_bias,
+                             window, causal, sm_scale, layout, out, ws, stream, "kessie_fog_prefill_varlen")
 
 
 def fog_prefill_batch(q: torch.Tensor, query_start_loc: torch.Tensor, max_query_len: int, pool: torch.Tensor,
@@ -321,15 +328,10 @@ def fog_prefill_batch(q: torch.Tensor, query_start_loc: torch.Tensor, max_query_
                       fog_vscale: Optional[torch.Tensor] = None, fog_bias: Optional[torch.Tensor] = None,
                       window: int = 0, causal: bool = True, sm_scale: Optional[float] = None,
                       layout: str = "native", out: Optional[torch.Tensor] = None,
-                      ws: Optional[torch.Tensor] = None, stream=None) -> bool:
+                      ws: Optional[torch.Tensor] = None, stream=None,
+                      entry: str = "kessie_fog_prefill_batch") -> bool:
     """fog_prefill_varlen for every shape of the MFMA kernels: also head_dim 64 and GQA ratios up to 16 that are no
     power of two (bf16/fp16), for which fog_prefill_varlen returns False."""
-    return _prefill_varlen("kessie_fog_prefill_batch", q, query_start_loc, max_query_len, pool, page_table, ctx_lens,
-                           max_ctx, fog_vscale, fog_bias, window, causal, sm_scale, layout, out, ws, stream)
-
-
-def _prefill_varlen(entry, q, query_start_loc, max_query_len, pool, page_table, ctx_lens, max_ctx, fog_vscale,
-                    fog_bias, window, causal, sm_scale, layout, out, ws, stream) -> bool:
     pv = pool_view(pool, layout)
     q = _contig(q, "q")
     t, hq, d = q.shape

@@ -63,3 +63,31 @@ def test_decode_known_lengths(dev, b, hq, hkv, d, dt, ctx, window, total):
         # One rounding of the output apart: only the splits' fp32 sums meet in another order.
         tol = {torch.bfloat16: 2 ** -7, torch.float16: 2 ** -10, torch.float32: 2e-5}[dt]
         assert bool((diff <= tol * (plain.float().abs() + 0.02)).all()), diff.max().item()
+
+
+def test_layer_passes_the_lengths_of_each_step(dev, monkeypatch):
+    """The serving layer's total of the lengths follows a metadata object that is refilled in place between steps, and a
+    window; it is left out of steps too small for it and with the fog off."""
+    from kessie_amd import kessie_attention as ka
+    from kessie_amd import ops
+
+    n, got = 4, []
+    q, pool, table, lens = decode_case(n, 8, 2, 64, 16384, 16, torch.bfloat16, dev, seed=45)
+    cache = pool.transpose(1, 2).contiguous()  # [pages, 2, page, heads, d]
+    cpu, qsl = lens.cpu(), torch.arange(n + 1, dtype=torch.int32)
+    meta = ka.KeSSieAttentionMetadata(n, 1, qsl.to(dev), 16384, lens, table, torch.zeros(n, dtype=torch.int64, device=dev),
+                                      query_start_loc_cpu=qsl, seq_lens_cpu=cpu)
+    real, state = ops.fog_decode, ka.KeSSieAttentionState()
+    monkeypatch.setattr(ops, "fog_decode", lambda *a, **k: (got.append(k.get("seen_total", 0)), real(*a, **k))[1])
+    monkeypatch.setattr(ka, "KESSIE_STATE", state)
+    new = torch.zeros(n, 2, 64, dtype=torch.bfloat16, device=dev)
+    for alpha, window, lengths in ((0.5, 0, [16384, 100, 40, 9]), (0.5, 0, [640, 200, 40, 9]),
+                                   (0.5, 13000, [16384, 200, 40, 9]), (0.5, 64, [640, 200, 40, 9]), (0.0, 0, [640, 200, 40, 9])):
+        state.update(fog_alpha=alpha, fog_start=0.5, prompt_len=16384)
+        cpu.copy_(torch.tensor(lengths))
+        lens.copy_(cpu)
+        impl = ka.KeSSieAttentionImpl(8, 64, 0.125, 2, sliding_window=window or None)
+        for _ in range(2):
+            impl.forward(None, q, new, new, cache, meta)
+    torch.cuda.synchronize()
+    assert got == [16533] * 2 + [889] * 2 + [13249] * 2 + [0] * 2 + [0] * 2
