@@ -2257,6 +2257,7 @@ static int prefill_varlen_entry(const void* q, const int32_t* query_start_loc, i
   using namespace kessie;
   using namespace kessie::attn;
   clear_error();
+  const char* name = any_shape ? "fog prefill batch" : "fog prefill varlen";
   Params p{};
   const int es = dtype_size(dtype);
   p.q = q;
@@ -2293,17 +2294,17 @@ static int prefill_varlen_entry(const void* q, const int32_t* query_start_loc, i
   p.sm_scale = sm_scale;
   int st = validate_common(p, dtype);
   if (st != KESSIE_OK) return st;
-  KESSIE_REQUIRE(max_query_len >= 0, KESSIE_ERR_INVALID, "fog prefill varlen: max_query_len %d", max_query_len);
+  KESSIE_REQUIRE(max_query_len >= 0, KESSIE_ERR_INVALID, "%s: max_query_len %d", name, max_query_len);
   KESSIE_REQUIRE(page_table != nullptr && ctx_lens != nullptr && query_start_loc != nullptr, KESSIE_ERR_INVALID,
-                 "fog prefill varlen: page_table, ctx_lens and query_start_loc are required");
-  KESSIE_REQUIRE(kv_stride >= 0, KESSIE_ERR_INVALID, "fog prefill varlen: kv_stride %lld", (long long)kv_stride);
+                 "%s: page_table, ctx_lens and query_start_loc are required", name);
+  KESSIE_REQUIRE(kv_stride >= 0, KESSIE_ERR_INVALID, "%s: kv_stride %lld", name, (long long)kv_stride);
   if (batch == 0 || max_query_len == 0) return KESSIE_OK;
   if (prefill_f32_ok(p, dtype)) return run_prefill_f32(p, workspace, workspace_bytes, stream);
   const bool listed = p.D == 128 && (p.G & (p.G - 1)) == 0;
   KESSIE_REQUIRE((any_shape || listed) && prefill_mfma_ok(p, dtype), KESSIE_ERR_UNSUPPORTED,
-                 "fog prefill varlen: shape not taken by the MFMA kernels (bf16/fp16: head_dim 128, pages of 16*2^k "
-                 "tokens, GQA 1/2/4/8/16; fp32: head_dim 128, pages of 16*2^k tokens, GQA up to 128; 16-byte aligned "
-                 "rows)");
+                 "%s: shape not taken by the MFMA kernels (bf16/fp16: head_dim 128%s, pages of 16*2^k tokens, GQA %s, "
+                 "sm_scale > 0; fp32: head_dim 128, pages of 16*2^k tokens, GQA up to 128; 16-byte aligned rows)",
+                 name, any_shape ? " or 64" : "", any_shape ? "up to 16" : "1/2/4/8/16");
   return run_prefill_mfma(p, dtype, workspace, workspace_bytes, stream);
 }
 

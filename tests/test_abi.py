@@ -129,6 +129,14 @@ def test_prefill_and_decode_argument_errors_without_gpu():
                                        None, 0, None, 0, fake, 2, 32, 8, 64, 16, 1024, 0, 0.125, 1, bf16,
                                        None, 0, None)
     assert st == _lib.ERR_UNSUPPORTED
+    assert "GQA 1/2/4/8/16" in _lib.last_error()[1]
+    # batch: 12-token pages are not, and the message is its own
+    st = lib.kessie_fog_prefill_batch(fake, fake, 64, fake, 1024, 32768, 2048, 1024, 64, fake, 64, fake,
+                                      None, 0, None, 0, fake, 2, 32, 8, 64, 12, 600, 0, 0.125, 1, bf16,
+                                      None, 0, None)
+    status, msg = _lib.last_error()
+    assert st == status == _lib.ERR_UNSUPPORTED
+    assert "fog prefill batch" in msg and "128 or 64" in msg and "GQA up to 16" in msg
     # paged prefill: a 64-query chunk on 64K keys splits the key range and needs a workspace
     need = lib.kessie_fog_prefill_workspace_bytes(1, 64, 32, 8, 128, 65536, 16, bf16)
     assert need > 0
