@@ -485,14 +485,15 @@ inline int combine_dsplit(int64_t rows, int D) {
 // decode's combine is latency-bound).  A balanced row's place among the units
 // is found by every wave for itself, without a barrier, and its splits past
 // the first kAheadLoads of a group are read in a loop (12 sequences of 3,000
-// in a balanced step: 34.3 -> 33.8 us).
+// in a balanced step: 34.3 -> 33.8 us).  An instance of its own: in one with the
+// plain rows it cost them 0.2 us (27 sequences of 466: 16.4 -> 16.1 us).
 // The same arithmetic in the same order as combine_kernel's fast path -- max
 // and sum over lanes s, s + 64, ... then the same butterfly, each group's
 // splits summed in increasing order, the groups met by the same sum_groups --
 // so the two give the same bits.
 constexpr int kAheadLoads = 8;
 
-template <typename T, bool TREE>
+template <typename T, bool TREE, bool kBalanced>
 __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p) {
   __shared__ float e_s[256];
   __shared__ float2 part[kCombineThreads];
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
   i += p.q0_off;
   const int tid = threadIdx.x, lane = tid & 63;
   int64_t first = row * S;
-  if (p.balanced) {
+  if constexpr (kBalanced) {
     const BatchPages bp = batch_pages(p);
     const int P = decode_unit_pages(bp, p.units, p.B);
     int u0;
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
       ay += e * v[j].y;
     }
   }
-  for (int sp = grp + kAheadLoads * groups; sp < S; sp += groups) {  // (balanced rows only)
+  for (int sp = grp + kAheadLoads * groups; kBalanced && sp < S; sp += groups) {
     const float e = e_s[sp];
     const float2 w = *reinterpret_cast<const float2*>(o + (int64_t)sp * D);
     ax += e * w.x;
@@ -596,8 +597,10 @@ void launch_row_combine(const Params& p, int64_t rows, hipStream_t s) {
   const int S = p.num_splits;
   bool ahead = (p.balanced ? p.units : S) <= 256 && (chunk & 1) == 0 && kCombineThreads % (chunk / 2) == 0;
   if (ahead && !p.balanced) ahead = S <= (kCombineThreads / (chunk / 2)) * kAheadLoads;
-  if (ahead)
-    hipLaunchKernelGGL((combine_ahead_kernel<T, TREE>), dim3((unsigned)rows, y), dim3(kCombineThreads), 0, s, p);
+  if (ahead && p.balanced)
+    hipLaunchKernelGGL((combine_ahead_kernel<T, TREE, true>), dim3((unsigned)rows, y), dim3(kCombineThreads), 0, s, p);
+  else if (ahead)
+    hipLaunchKernelGGL((combine_ahead_kernel<T, TREE, false>), dim3((unsigned)rows, y), dim3(kCombineThreads), 0, s, p);
   else
     hipLaunchKernelGGL((combine_kernel<T, TREE>), dim3((unsigned)rows, y), dim3(kCombineThreads), 0, s, p);
 }
