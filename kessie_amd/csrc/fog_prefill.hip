@@ -568,28 +568,35 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
           kScaleV ? pack2<T>(to_f32(a) * fw0[set], to_f32(b) * fw1[set]) : bits16(a) | (bits16(b) << 16);
     }
   };
-  auto store_rows = [&](int t, int set) {  // tile t's K rows, bias and weights
+  auto v_dst = [&](int t) { return vts + v_stage(t) + 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3); };
+  auto store_k = [&](int t, int set) {
     T* kd = ks + k_stage(t) + 8 * kc;
 #pragma unroll
     for (int r = 0; r < kKL; ++r) *reinterpret_cast<v8*>(kd + krow_lds(r) * kKRow) = kreg[set][r];
+  };
+  auto store_fog = [&](int t, int set) {
     if (kBias && tid < kPfKT) fbs[f_stage(t) + tid] = base2_bias(fb_r[set]);
     if (kVs && kExactP && tid < kPfKT) fws[f_stage(t) + tid] = fk_r[set];
   };
-  const int v_at0 = 4 * ((kp >> 2) ^ (kc >> 1)) + (kp & 3);
-  auto store = [&](int t, int set) {
-    store_rows(t, set);
+  auto store = [&](int t, int set) {  // tile t into its stages
+    store_k(t, set);
     if (vload) {
+      uint32_t* vd = v_dst(t);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) store_v(vts + v_stage(t) + v_at0, e, set);
+      for (int e = 0; e < 8; ++e) store_v(vd, e, set);
     }
+    store_fog(t, set);
   };
 
   // Slice i of n (n >= 8) of store(): V^T word i for i < 8, then the K rows
   // and the bias at slice n-1 -- spread over the PV MFMAs.  With no tile
   // t+2 it rewrites a stage that no later tile reads.
   auto store_slice = [&](int t, int i, int n, int set) {
-    if (vload && i < 8) store_v(vts + v_stage(t) + v_at0, i, set);
-    if (i == n - 1) store_rows(t, set);
+    if (vload && i < 8) store_v(v_dst(t), i, set);
+    if (i == n - 1) {
+      store_k(t, set);
+      store_fog(t, set);
+    }
   };
   // S^T of the tile in a stage: lane (col, half) reads K row 32kb + col.
   const T* kread = ks + col * kKRow + 8 * half;
