@@ -1377,17 +1377,42 @@ int decode_splits(int B, int Hkv, int max_ctx, int page_size, int target = decod
 // sequences on a 4,096-token window 62.6 -> 46.8.  A window bounds the blocks
 // there are to split: decode_splits leaves a short window's splits mostly
 // empty (4 sequences, 1 kv head, window 1,024: 15.5 -> 14.4 us).
-// target: decode_target(); bound: decode_splits.
-int decode_launch_splits(int B, int Hkv, int max_ctx, int window, int page_size, int target, int bound) {
+// Rounded up where the longer splits cost more than the second round (graph
+// replays; both ways):
+//   * a surplus of 1/64 of the round or less against splits a third longer (12
+//     sequences, 1 kv head, window 4,096, 3 and 4 blocks: 18.0 and 19.0 us);
+//   * fp32, whose surplus workgroups run faster beside fewer others: up to 1/10
+//     against splits 1/8 longer (24 sequences of 140-700 37.1 and 38.6 us, 40 of
+//     60-300 29.6 and 31.5, of 140-700 53.4 and 56.1; equal ones of 700 79.4 and
+//     80.5, of 300 44.3 and 42.6);
+//   * more than kBalSeqs sequences, which cannot share their units by pages,
+//     unless they are known to be of about one length (90 of 1,000-5,000 210 and
+//     231 us, equal 381 and 289).
+// (Mixed lengths of a few sequences that the host does not know lose up to 4 %
+// by rounding down, 12 of 300-1,500 18.8 and 19.6 us, where equal ones gain: 24
+// of 1,500 37.1 and 33.0.)
+// seen_total: decode_entry's; target: decode_target(); bound: decode_splits.
+int decode_launch_splits(int B, int Hkv, int max_ctx, int window, int page_size, int dtype, int64_t seen_total,
+                         int target, int bound) {
   const int units = max(B * div_up(Hkv, kDecWaves), 1);
+  const int blk = max(min(page_size, 16), 1);
+  const bool windowed = window > 0 && window < max_ctx;
+  const int blocks = windowed ? div_up(window, blk) + 1 : div_up(max(max_ctx, 1), blk);
+  const int up = div_up(target, units);
   int s = target / units;
   // Past half a round of units there is no second split to round down to: two
   // splits, whose surplus fills in behind sequences that end early.
-  if (s < 2) s = div_up(target, units);
-  if (window > 0 && window < max_ctx) {
-    const int blk = max(min(page_size, 16), 1);
-    s = min(s, (div_up(window, blk) + 1) / 2);
+  if (s < 2) {
+    s = up;
+  } else if (up > s) {
+    const int64_t surplus = (int64_t)up * units - target;
+    const int64_t per_up = div_up(blocks, up), per = div_up(blocks, s);
+    const bool one_length = 20.0 * (double)seen_total >= 17.0 * B * (windowed ? window : max_ctx);
+    if ((64 * surplus <= target && 4 * per_up <= 3 * per) ||
+        (dtype == KESSIE_DTYPE_F32 && 10 * surplus <= target && 9 * per_up <= 8 * per) || (B > kBalSeqs && !one_length))
+      s = up;
   }
+  if (windowed) s = min(s, (div_up(window, blk) + 1) / 2);
   return max(1, min(s, bound));
 }
 
@@ -1915,7 +1940,7 @@ static int decode_entry(const void* q, const void* kv_pool, int num_pages, int64
   if (decode_mfma_ok(p, dtype)) {
     // The partials-only form and the generic kernel keep the bound's splits.
     if (!partials_only && !p.direct_out) {
-      p.num_splits = decode_launch_splits(batch, num_kv_heads, max_ctx, window, page_size, target, bound);
+      p.num_splits = decode_launch_splits(batch, num_kv_heads, max_ctx, window, page_size, dtype, seen_total, target, bound);
       p.direct_out = p.num_splits == 1 ? 1 : 0;
     }
     // Split partials merged here: assign the splits by pages across the batch

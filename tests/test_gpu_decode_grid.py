@@ -19,6 +19,8 @@ pytestmark = pytest.mark.gpu
     (4, 1, 9000, [9000, 8999, 33, 1], 33),                  # ... to two of them
     (3, 1, 4000, [4000, 40, 17], 5),                        # ... and to one (no partials)
     (130, 8, 64, [64] * 100 + [1 + i for i in range(30)], 0),  # past half a round: two splits
+    (12, 1, 5000, [5000] * 11 + [77], 4096),                # rounded up: few surplus workgroups
+    (70, 8, 500, [500] * 3 + [7 * i + 1 for i in range(67)], 0),  # rounded up: a large batch of unknown lengths
 ])
 def test_decode_one_round_grid(dev, b, hkv, ctx, lens, window):
     from kessie_amd import ops
@@ -41,7 +43,9 @@ def test_decode_one_round_grid(dev, b, hkv, ctx, lens, window):
 
 @pytest.mark.parametrize("b,hq,hkv,d,dt,ctx,window", [
     (12, 32, 8, 128, torch.bfloat16, 3000, 0), (12, 32, 8, 64, torch.float16, 6000, 0),
-    (24, 8, 2, 128, torch.float32, 4000, 0), (24, 24, 8, 128, torch.bfloat16, 2000, 1000),
+    (24, 8, 2, 128, torch.float32, 4000, 0), (40, 32, 8, 128, torch.float32, 300, 0),  # fp32: rounded up
+    (70, 32, 8, 128, torch.bfloat16, 500, 0),  # rounded up, or down by the total
+    (24, 24, 8, 128, torch.bfloat16, 2000, 1000),
     (20, 32, 2, 128, torch.bfloat16, 9000, 0),  # 1,024 units a group of heads: the combine that loops
 ])
 @pytest.mark.parametrize("total", ["sum", "one", "over"])
