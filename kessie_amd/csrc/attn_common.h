@@ -60,11 +60,10 @@ struct Params {
   int direct_out;      // 1: the main kernel writes the normalised output
   int launch_combine;  // host side: follow the main kernel with the combine
   int balanced;        // decode split partials: units assigned by pages (decode_seq_of_unit)
+  int units;           // workgroups per group of kv heads of a balanced decode
   float* ws_o;  // [B*C*Hq][S][D]
   float* ws_m;  // [B*C*Hq][S]
   float* ws_l;  // [B*C*Hq][S]
-  int units;    // workgroups per group of kv heads of a balanced decode (last: the
-                // other fields' places are what the short decodes' loads were timed with)
 };
 
 // A sequence length as the kernels use it: at most max_ctx and the page
