@@ -485,7 +485,8 @@ inline int combine_dsplit(int64_t rows, int D) {
 // decode's combine is latency-bound).  A balanced row's place among the units
 // is found by every wave for itself, without a barrier, and its splits past
 // the first kAheadLoads of a group are read in a loop (12 sequences of 3,000
-// in a balanced step: 34.3 -> 33.8 us).  An instance of its own: in one with the
+// in a balanced step: 34.3 -> 33.8 us), eight at a time: one at a time held the
+// long rows up (2 x 131,072 + 14 x 4,096: 9.6 us, 6.8 so, combine_kernel 8.3).  An instance of its own: in one with the
 // plain rows it cost them 0.2 us (27 sequences of 466: 16.4 -> 16.1 us).
 // The same arithmetic in the same order as combine_kernel's fast path -- max
 // and sum over lanes s, s + 64, ... then the same butterfly, each group's
@@ -572,6 +573,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_ahead_kernel(Params p
       ay += e * v[j].y;
     }
   }
+#pragma unroll 8
   for (int sp = grp + kAheadLoads * groups; kBalanced && sp < S; sp += groups) {
     const float e = e_s[sp];
     const float2 w = *reinterpret_cast<const float2*>(o + (int64_t)sp * D);
