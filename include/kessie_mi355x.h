@@ -276,8 +276,8 @@ int kessie_fog_prefill_varlen(
 
 /* kessie_fog_prefill_varlen for every shape of the MFMA kernels: also head_dim
  * 64 and GQA ratios up to 16 that are no power of two (bf16/fp16), which the
- * other entry reports as unsupported.  Same arguments, semantics and
- * workspace. */
+ * other entry reports as unsupported (its callers, who run those per sequence,
+ * were promised that).  Same arguments, semantics and workspace. */
 int kessie_fog_prefill_batch(
     const void* q, const int32_t* query_start_loc, int max_query_len,
     const void* kv_pool, int num_pages, int64_t page_stride, int64_t tok_stride,

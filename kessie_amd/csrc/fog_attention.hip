@@ -23,7 +23,7 @@
 //   attn_generic  any dtype / head_dim <= 256 / page size / GQA ratio: K and
 //                 V tiles staged in LDS as fp32, one workgroup per
 //                 (row tile, kv head, sequence, split).  Serves the shapes the
-//                 MFMA kernels do not take (fp32 prefill, other head_dims,
+//                 MFMA kernels do not take (fp32 at head_dim 64, other head_dims,
 //                 page sizes and GQA ratios).
 //   combine       merges the per-split (m, l, o) partials of either kernel.
 #include <climits>
@@ -1432,7 +1432,8 @@ dim3 decode_grid(const Params& p) {
 }
 
 // Key splits of the MFMA prefill: enough workgroups for one per CU (one fits a
-// CU at a time: 106.5 KiB of LDS), at least 8 key tiles (512 keys) per split.
+// CU at a time: eight waves of 188-256 VGPRs, and at head_dim 128 149 KiB of
+// LDS), at least 8 key tiles (512 keys) per split.
 // A 2,048-query chunk at GQA 4 and 8 kv heads already has 256 workgroups: no
 // split.  Under causal masking the chunk's query tiles see max_ctx - C/2 keys
 // on average (half the context for a fresh prompt), and the per-split minimum
@@ -2022,8 +2023,8 @@ extern "C" int kessie_fog_decode_partials(const void* q, const void* kv_pool, in
 // of the array, at its own address, until the process ends; host code uses
 // that address (from hipGetSymbolAddress, once per device), never the array's
 // name.  Calls that overlap on one GPU share the array and race.  The decode
-// kernels write every partial of every (row, split) on each call, so nothing
-// needs clearing between calls.
+// kernels write every partial that their combine reads on each call (balanced:
+// the units in use), so nothing needs clearing between calls.
 // ---------------------------------------------------------------------------
 namespace {
 static __device__ __align__(256) unsigned char scratch[KESSIE_DECODE_NOALLOC_SCRATCH_BYTES];
@@ -2369,7 +2370,8 @@ extern "C" int kessie_fog_prefill_batch(const void* q, const int32_t* query_star
 }
 
 // Reference launchers (kessie_kernels_v2.hip:716-751, 788-825): dense fp16
-// [B,H,N,D], no GQA, every position a query.  One split, so no workspace.
+// [B,H,N,D], no GQA, every position a query.  They take no workspace: split
+// partials go to a buffer of the library's (dense_workspace).
 namespace kessie {
 namespace attn {
 namespace {
@@ -2416,7 +2418,13 @@ int dense_splits(int B, int H, int N, int window, int causal, int* split_q0) {
   // 2, 4, 8) the best were 2 where the longest tile is 1.9-3.8 times the
   // share (N=4,096-8,192 full, N=4,096 W=1,024) and 4 from 5.3 times on
   // (N=512-2,048, full and W=1,024), down to 2 key tiles per split (N=512:
-  // 22.4 us against 24.1 with 4 tiles per split).
+  // 22.4 us against 24.1 with 4 tiles per split).  At head_dim 64 and with
+  // kExactP the same counts are the best or within 3 % (1, 2, 3, 4, 6, 8: H=8
+  // D=64 N=1,024 29.9, 25.3, 23.8, 21.6, 22.6, 22.8 us, N=8,192 179, 129, 159,
+  // 142, 159, 173; kExactP H=12 N=1,001 38.5, 31.4, 28.9, 26.6, 29.1, 32.6,
+  // D=128 N=5,001 245, 190, 219, 210, 234, 265), but for kExactP at N=2,001,
+  // where 3 takes 42.5 us against 47.7 (D=64) and 59.6 against 70 (D=128), and
+  // for 4 x 12 x 1,001 x 128 without fog, where 1 takes 59 against 80.
   const double ratio = longest / share;
   if (ratio < 1.5) return 1;
   int s = ratio >= 5.0 ? 4 : 2;
