@@ -715,7 +715,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(Params p) {
     // the matrix pipe busy while its VALU works.
     // (kExactP at head_dim 128, whose probabilities' second operands have no
     // registers left, runs as two halves of 32 keys: the QK steps of one score
-    // block with this half's exponentials, then the half's PV steps.  28-89
+    // block with this half's exponentials, then the half's PV steps.  22-89
     // VGPRs spilled otherwise; 2,048 bf16 queries on 16,384, 24 q / 8 kv, 746 ->
     // 637 us, with V weights on 32-token pages 1,209 -> 789.  At head_dim 64,
     // which spills nothing, it costs 3 %.)
